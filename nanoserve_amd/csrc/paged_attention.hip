@@ -26,8 +26,8 @@
 //     The hand-off uses agent-scope atomic stores/loads and a store-completion wait before the counter
 //     (ns_common.h, publish_*), not device-scope fences, which on gfx950 write back and invalidate the
 //     XCD's whole L2 in every workgroup.
-// fp32 design: one wave per (row, KV head), VALU dot products with wave reductions; kept simple,
-// it serves the fp32 correctness paths.
+// fp32 design (the correctness configuration): one workgroup per (row, KV head), VALU products with one lane per
+// token for the scores and one lane per dim for P.V (paged_decode_f32_kernel).
 #include "ns_common.h"
 #include "prefill_body.h"
 
@@ -878,64 +878,195 @@ __global__ __launch_bounds__(PF_WG_THREADS) __attribute__((amdgpu_waves_per_eu(2
     decode_rows_body<HD, PH>(ra, int(blockIdx.x) - n_pf, lds, sm_m, sm_l, s_last);
 }
 
-// fp32: one wave per (row, KV head). Lane owns dims lane and lane + 64 (hd 128).
-template <int HD>
-__global__ __launch_bounds__(64) void paged_decode_f32_kernel(
+// fp32: one workgroup per (row, KV head); its waves take 64-token chunks in turn. Where a row has fewer chunks
+// than waves, several waves share a chunk and split its query heads (wave w of a workgroup runs on SIMD w, so
+// with whole chunks per wave the short rows of a prompt would all queue on the first SIMDs of a CU).
+//   * Scores: four lanes per token, each with a quarter of its dims, so a load instruction reads 64 bytes of 16
+//     token rows, and a score is the sum over four neighbouring lanes; each of the four keeps another page's, so
+//     the online-softmax statistics cost one wave maximum per head and 64 tokens. Queries sit in LDS.
+//   * P.V: lane = dim (lane and lane + 64 for hd 128). A V row is one coalesced load; the weights come back
+//     from LDS, four tokens per read.
+//   * The waves' states (m, l, acc) merge through LDS in wave order; a row's result does not depend on the grid.
+// It serves the fp32 correctness configuration, whose prompts run as one row per token, so rows are many and
+// short. Bound by latency (block ids -> K / V rows) and the vector ALUs: 4 x 128-token prompts of 14 / 2 heads
+// of 64 take 19 us a call; the earlier kernel (one wave per row and KV head, a token and a 6-step wave sum at a
+// time) took 296 us.
+// K rows load 16 bytes per lane where pointer and strides allow it (VEC), else dword by dword: fp32 callers have
+// never been held to an alignment. GC: query heads per KV head the registers hold (8 or 16).
+constexpr int F32_NW = 4, F32_CH = 64;
+template <int HD, int GC, bool VEC>
+__global__ __launch_bounds__(F32_NW * 64) void paged_decode_f32_kernel(
     const float* __restrict__ q, int64_t q_sb, int64_t q_sh, const float* __restrict__ kp,
     const float* __restrict__ vp, int64_t s_blk, int64_t s_pos, int64_t s_h, const int32_t* __restrict__ bt,
     int64_t bt_sb, const int32_t* __restrict__ ctxl, float* __restrict__ out, int64_t o_sb, int64_t o_sh, int G,
     int max_blocks, int num_blocks, float scale, const int64_t* __restrict__ qrows) {
-  constexpr int DL = HD / 64;  // dims per lane
-  const int g = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
+  constexpr int DL = HD / 64;                  // dims per lane in P.V
+  constexpr int PG = F32_CH / PAGE;            // pages per chunk
+  __shared__ __align__(16) float sq[GC * HD];
+  __shared__ __align__(16) float sp[F32_NW][GC * F32_CH];   // a chunk's weights; at the end the waves' (m, l)
+  __shared__ float sacc[F32_NW][GC * HD];
+  const int g = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t qb = qrows != nullptr ? qrows[b] : int64_t(b);   // q / out row of entry b
   const int ctx = ctxl[b];
   int n_pages = ctx > 0 ? (ctx + PAGE - 1) / PAGE : 0;
   if (n_pages > max_blocks) n_pages = max_blocks;
   const int n_tok = ctx < n_pages * PAGE ? ctx : n_pages * PAGE;
-  float qv[16][DL], acc[16][DL], m[16], l[16];
+  float* orow = out + qb * o_sb + int64_t(g) * G * o_sh;
+  if (n_tok <= 0) {   // no keys: zeros (the whole workgroup leaves)
+    for (int i = tid; i < G * HD; i += F32_NW * 64) orow[int64_t(i / HD) * o_sh + i % HD] = 0.f;
+    return;
+  }
+  for (int i = tid; i < G * HD; i += F32_NW * 64) sq[i] = q[qb * q_sb + int64_t(g * G + i / HD) * q_sh + i % HD];
+  __syncthreads();
+
+  const int n_ch = (n_tok + F32_CH - 1) / F32_CH;
+  const int hs = n_ch >= 3 ? 1 : n_ch == 2 ? 2 : F32_NW;   // waves that share a chunk
+  const int hg = w & (hs - 1);                             // this wave's heads: h % hs == hg
+  float m[GC], l[GC], acc[GC][DL];
 #pragma unroll
-  for (int h = 0; h < 16; ++h) {
+  for (int h = 0; h < GC; ++h) {
     m[h] = -INFINITY;
     l[h] = 0.f;
 #pragma unroll
-    for (int e = 0; e < DL; ++e) {
-      qv[h][e] = h < G ? q[qb * q_sb + int64_t(g * G + h) * q_sh + lane + 64 * e] : 0.f;
-      acc[h][e] = 0.f;
-    }
+    for (int e = 0; e < DL; ++e) acc[h][e] = 0.f;
   }
-  for (int t = 0; t < n_tok; ++t) {
-    const int blk = bt[int64_t(b) * bt_sb + t / PAGE];
-    const bool ok = blk >= 0 && blk < num_blocks;
-    const int64_t off = int64_t(ok ? blk : 0) * s_blk + int64_t(t % PAGE) * s_pos + int64_t(g) * s_h;
-    float kv[DL], vv[DL];
+  for (int c = w / hs; c < n_ch; c += F32_NW / hs) {
+    // block ids: lane p < PG holds the chunk's page p's. A block outside the pool is read as zero rows.
+    const int t0 = c * F32_CH;
+    const int blk = bt[int64_t(b) * bt_sb + min(t0 / PAGE + (lane & (PG - 1)), n_pages - 1)];
+    const bool blk_ok = blk >= 0 && blk < num_blocks;
+    // K: lane 4 t + d reads, of every page's token t, dims 16 i + 4 d .. + 3
+    float4_t kr[PG][HD / 16];
 #pragma unroll
-    for (int e = 0; e < DL; ++e) {
-      kv[e] = ok ? kp[off + lane + 64 * e] : 0.f;
-      vv[e] = ok ? vp[off + lane + 64 * e] : 0.f;
-    }
+    for (int pg = 0; pg < PG; ++pg) {
+      const float* krow = kp + int64_t(__builtin_amdgcn_readlane(blk_ok ? blk : 0, pg)) * s_blk +
+                          int64_t(lane >> 2) * s_pos + int64_t(g) * s_h + 4 * (lane & 3);
 #pragma unroll
-    for (int h = 0; h < 16; ++h) {
-      if (h < G) {
-        float part = 0.f;
+      for (int i = 0; i < HD / 16; ++i) {
+        if constexpr (VEC) {
+          kr[pg][i] = *reinterpret_cast<const float4_t*>(krow + 16 * i);
+        } else {
 #pragma unroll
-        for (int e = 0; e < DL; ++e) part = fmaf(qv[h][e], kv[e], part);
-        const float s = wave_sum(part) * scale;
-        const float m_new = fmaxf(m[h], s);
-        const float alpha = expf(m[h] - m_new);
-        const float p = expf(s - m_new);
-        l[h] = l[h] * alpha + p;
-#pragma unroll
-        for (int e = 0; e < DL; ++e) acc[h][e] = acc[h][e] * alpha + p * vv[e];
-        m[h] = m_new;
+          for (int e = 0; e < 4; ++e) kr[pg][i][e] = krow[16 * i + e];
+        }
       }
     }
+    // V rows of one page, a lane's dims of each (pages past the row's end re-read its last one: never used)
+    float v[2][PAGE][DL];
+    auto load_v = [&](int pg, float (&dst)[PAGE][DL]) __attribute__((always_inline)) {
+      const float* vbase = vp + int64_t(__builtin_amdgcn_readlane(blk_ok ? blk : 0, pg)) * s_blk + int64_t(g) * s_h;
+#pragma unroll
+      for (int t = 0; t < PAGE; ++t)
+#pragma unroll
+        for (int e = 0; e < DL; ++e) dst[t][e] = vbase[int64_t(t) * s_pos + lane + 64 * e];
+    };
+    load_v(0, v[0]);
+    __builtin_amdgcn_sched_barrier(0);   // both loads go out before the scores wait for the first
+    // lane 4 t + d keeps the score of token t of page d
+    const int my_tok = PAGE * (lane & 3) + (lane >> 2);
+    const bool live = t0 + my_tok < n_tok;
+    const bool tok = __shfl(int(blk_ok), lane & 3, 64) != 0;
+#pragma unroll
+    for (int h = 0; h < GC; ++h) {
+      if (h < G && (h & (hs - 1)) == hg) {
+        float part[PG];
+#pragma unroll
+        for (int pg = 0; pg < PG; ++pg) part[pg] = 0.f;
+#pragma unroll
+        for (int i = 0; i < HD / 16; ++i) {
+          const float4_t qv = *reinterpret_cast<const float4_t*>(sq + h * HD + 16 * i + 4 * (lane & 3));
+#pragma unroll
+          for (int pg = 0; pg < PG; ++pg)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[pg] = fmaf(qv[e], kr[pg][i][e], part[pg]);
+        }
+        // sums over the token's four lanes
+        float s = 0.f;
+#pragma unroll
+        for (int pg = 0; pg < PG; ++pg) {
+          part[pg] += __shfl_xor(part[pg], 1, 64);
+          part[pg] += __shfl_xor(part[pg], 2, 64);
+          s = (lane & 3) == pg ? part[pg] : s;
+        }
+        s = tok ? s * scale : 0.f;
+        const float m_new = fmaxf(m[h], wave_max(live ? s : -INFINITY));
+        const float p = live ? expf(s - m_new) : 0.f;
+        const float alpha = expf(m[h] - m_new);
+        l[h] = l[h] * alpha + p;   // this lane's tokens; summed over the lanes at the end
+#pragma unroll
+        for (int e = 0; e < DL; ++e) acc[h][e] *= alpha;
+        m[h] = m_new;
+        sp[w][h * F32_CH + my_tok] = p;
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave's weights are in LDS (no other wave reads them)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+#pragma unroll
+    for (int pg = 0; pg < PG; ++pg) {
+      const int n_here = n_tok - t0 - PAGE * pg;   // tokens of this page that exist (wave-uniform)
+      if (n_here <= 0) break;
+      if (pg + 1 < PG) load_v(pg + 1, v[(pg + 1) & 1]);   // in flight while this page multiplies
+      const bool ok = __builtin_amdgcn_readlane(int(blk_ok), pg) != 0;
+#pragma unroll
+      for (int t = 0; t < PAGE; ++t)   // slots that hold no token, and blocks outside the pool, count as zeros
+#pragma unroll
+        for (int e = 0; e < DL; ++e) v[pg & 1][t][e] = ok && t < n_here ? v[pg & 1][t][e] : 0.f;
+#pragma unroll
+      for (int h = 0; h < GC; ++h) {
+        if (h < G && (h & (hs - 1)) == hg) {
+#pragma unroll
+          for (int t4 = 0; t4 < PAGE / 4; ++t4) {
+            const float4_t pv = *reinterpret_cast<const float4_t*>(&sp[w][h * F32_CH + PAGE * pg + 4 * t4]);
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+              for (int e = 0; e < DL; ++e) acc[h][e] = fmaf(pv[x], v[pg & 1][4 * t4 + x][e], acc[h][e]);
+          }
+        }
+      }
+    }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);   // the next chunk's weights stay behind these reads
   }
 #pragma unroll
-  for (int h = 0; h < 16; ++h)
-    if (h < G)
+  for (int h = 0; h < GC; ++h) {
+    if (h < G && (h & (hs - 1)) == hg) {
+      const float ls = wave_sum(l[h]);
+      if (lane == 0) {
+        sp[w][2 * h] = m[h];
+        sp[w][2 * h + 1] = ls;
+      }
 #pragma unroll
-      for (int e = 0; e < DL; ++e)
-        out[qb * o_sb + int64_t(g * G + h) * o_sh + lane + 64 * e] = n_tok > 0 ? acc[h][e] / l[h] : 0.f;
+      for (int e = 0; e < DL; ++e) sacc[w][h * HD + lane + 64 * e] = acc[h][e];
+    }
+  }
+  __syncthreads();
+  const int n_live = min(n_ch, F32_NW / hs);   // waves that had a chunk of a head: hg, hg + hs, ...
+  for (int i = tid; i < G * HD; i += F32_NW * 64) {
+    const int h = i / HD;
+    const int x0 = h & (hs - 1), x1 = x0 + n_live * hs;
+    float M = sp[x0][2 * h];
+    for (int x = x0 + hs; x < x1; x += hs) M = fmaxf(M, sp[x][2 * h]);
+    float L = 0.f, A = 0.f;
+    for (int x = x0; x < x1; x += hs) {
+      const float wgt = expf(sp[x][2 * h] - M);
+      L += wgt * sp[x][2 * h + 1];
+      A += wgt * sacc[x][i];
+    }
+    orow[int64_t(h) * o_sh + i % HD] = A / L;
+  }
+}
+
+template <int HD, int GC>
+static void launch_f32(bool vec, dim3 grid, hipStream_t s, const float* q, int64_t q_sb, int64_t q_sh, const float* kp,
+                       const float* vp, int64_t s_blk, int64_t s_pos, int64_t s_h, const int32_t* bt, int64_t bt_sb,
+                       const int32_t* ctxl, float* out, int64_t o_sb, int64_t o_sh, int G, int max_blocks, int num_blocks,
+                       float scale, const int64_t* qrows) {
+  if (vec)
+    hipLaunchKernelGGL((paged_decode_f32_kernel<HD, GC, true>), grid, dim3(F32_NW * 64), 0, s, q, q_sb, q_sh, kp, vp, s_blk,
+                       s_pos, s_h, bt, bt_sb, ctxl, out, o_sb, o_sh, G, max_blocks, num_blocks, scale, qrows);
+  else
+    hipLaunchKernelGGL((paged_decode_f32_kernel<HD, GC, false>), grid, dim3(F32_NW * 64), 0, s, q, q_sb, q_sh, kp, vp, s_blk,
+                       s_pos, s_h, bt, bt_sb, ctxl, out, o_sb, o_sh, G, max_blocks, num_blocks, scale, qrows);
 }
 
 static inline int decode_parts(int head_dim, int max_blocks) {
@@ -1035,16 +1166,12 @@ static int paged_decode_launch(const void* q, int64_t q_sb, int64_t q_sh, const 
   if (B == 0) return NS_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (dtype == NS_DTYPE_F32) {
-    if (head_dim == 64)
-      hipLaunchKernelGGL(paged_decode_f32_kernel<64>, dim3(n_kv_heads, B), dim3(64), 0, s,
-                         static_cast<const float*>(q), q_sb, q_sh, static_cast<const float*>(k_pool),
-                         static_cast<const float*>(v_pool), kv_sblk, kv_spos, kv_sh, block_tables, bt_sb, context_lens,
-                         static_cast<float*>(out), o_sb, o_sh, G, max_blocks, num_blocks, scale, qrows);
-    else
-      hipLaunchKernelGGL(paged_decode_f32_kernel<128>, dim3(n_kv_heads, B), dim3(64), 0, s,
-                         static_cast<const float*>(q), q_sb, q_sh, static_cast<const float*>(k_pool),
-                         static_cast<const float*>(v_pool), kv_sblk, kv_spos, kv_sh, block_tables, bt_sb, context_lens,
-                         static_cast<float*>(out), o_sb, o_sh, G, max_blocks, num_blocks, scale, qrows);
+    const bool vec = reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && kv_sblk % 4 == 0 && kv_spos % 4 == 0 && kv_sh % 4 == 0;
+    const auto launch = head_dim == 64 ? (G <= 8 ? launch_f32<64, 8> : launch_f32<64, 16>)
+                                       : (G <= 8 ? launch_f32<128, 8> : launch_f32<128, 16>);
+    launch(vec, dim3(n_kv_heads, B), s, static_cast<const float*>(q), q_sb, q_sh, static_cast<const float*>(k_pool),
+           static_cast<const float*>(v_pool), kv_sblk, kv_spos, kv_sh, block_tables, bt_sb, context_lens,
+           static_cast<float*>(out), o_sb, o_sh, G, max_blocks, num_blocks, scale, qrows);
     return check_launch("paged_attention_decode(f32)");
   }
   // bf16: 16-byte fragment loads need 8-element aligned strides and 16-byte aligned bases.
