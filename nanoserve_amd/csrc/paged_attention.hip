@@ -354,7 +354,7 @@ __global__ __launch_bounds__(DecodeCfg<HD>::NW * 64) void paged_decode_bf16_kern
 constexpr int ROWK_NW = 8, ROWK_PPW = 4, ROWK_D = 2, ROWK_PART = ROWK_NW * ROWK_PPW;
 constexpr int ROWK_MB = 8;
 constexpr int ROWK_VALU_G = 8, ROWK_VALU_G_PH = 6;   // query heads per KV head the VALU variant takes
-constexpr int ROWK_MAX_PARTS = 32;
+constexpr int ROWK_VALU_MAX_PARTS = 32;   // partitions the VALU variant takes
 typedef __attribute__((ext_vector_type(4))) unsigned int rk_u32x4_t;
 typedef __attribute__((ext_vector_type(2))) unsigned int rk_u32x2_t;
 
@@ -1079,14 +1079,18 @@ static inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 using namespace ns;
 
-// Whole-row kernel: n_kv * head_dim == 128 (one 256-byte token row), <= 16 query heads, token rows
-// contiguous in the pool, and a table width its merge covers.
 // KV heads that are workgroup rows of their own: 1 when a token's K row (all KV heads) is 256 bytes
-// (n_kv * head_dim == 128, token rows contiguous), n_kv for hd 128 with several KV heads (one head's 256
-// bytes per workgroup row, tokens kv_spos apart); 0 when the whole-row kernel does not apply.
+// (n_kv * head_dim == 128, token rows contiguous, at most 16 query heads), n_kv for hd 128 with several KV heads
+// (one head's 256 bytes per workgroup row, tokens kv_spos apart); 0 when the whole-row kernel does not apply.
+// It takes every table width that the per-head kernel accepts: its partitions are 32 pages against 8 (hd 128)
+// and 16 (hd 64), so long rows have a quarter of the states to merge, and its loads are whole lines. (12 rows of
+// 9k-29k tokens, 16 / 2 heads of 128: 100 us per layer on the per-head kernel, 62 us here.)
 static inline int rows_kernel_grid_heads(int n_heads, int n_kv_heads, int head_dim, int64_t kv_spos, int64_t kv_sh,
-                                         int max_blocks) {
-  if ((max_blocks + ROWK_PART - 1) / ROWK_PART > ROWK_MAX_PARTS) return 0;
+                                         int max_blocks, bool valu) {
+  const int widest = valu ? ROWK_VALU_MAX_PARTS * ROWK_PART
+                          : head_dim == 64 ? MERGE_MAX_PARTS<64> * DecodeCfg<64>::NW * DecodeCfg<64>::PPW
+                                           : MERGE_MAX_PARTS<128> * DecodeCfg<128>::NW * DecodeCfg<128>::PPW;
+  if (max_blocks > widest) return 0;
   if (n_kv_heads * head_dim == 128 && n_heads <= 16 && kv_sh == head_dim && kv_spos == 128) return 1;
   if (head_dim == 128 && n_kv_heads > 1 && n_heads / n_kv_heads <= 16 && kv_sh == 128 && kv_spos % 8 == 0)
     return n_kv_heads;
@@ -1183,7 +1187,7 @@ static int paged_decode_launch(const void* q, int64_t q_sb, int64_t q_sh, const 
                  0,
              "paged_attention_decode: q / k_pool / v_pool must be 16-byte aligned");
   const float sl2 = scale * LOG2E;
-  const int rgh = rows_kernel_grid_heads(n_heads, n_kv_heads, head_dim, kv_spos, kv_sh, max_blocks);
+  const int rgh = rows_kernel_grid_heads(n_heads, n_kv_heads, head_dim, kv_spos, kv_sh, max_blocks, valu);
   if (rgh > 0) {
     NS_REQUIRE(!valu || G <= (rgh > 1 ? ROWK_VALU_G_PH : ROWK_VALU_G),
                "paged_attention_decode_valu: GQA group %d above %d for this shape", G, rgh > 1 ? ROWK_VALU_G_PH : ROWK_VALU_G);

@@ -69,3 +69,19 @@ def test_fp32_rows_ignore_what_lies_past_the_context(hiplib):
     out = paged_attention_decode(q.cuda(), k.cuda(), v.cuda(), tables.cuda(), cl.cuda(), 0.125).cpu()
     assert (out[2] == 0).all()
     assert (out.double() - clean).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,width", [(16, 2, 128, 1024), (16, 2, 128, 1025), (12, 2, 128, 2048), (14, 2, 64, 1025),
+                                                   (14, 2, 64, 2049), (16, 1, 128, 2048)])
+def test_wide_tables(hiplib, n_heads, n_kv, hd, width):
+    """Tables of more than 32 partitions: rows that end in the first, a middle and the last partition. P is rounded to
+    bf16 before P.V and the output once more: 2^-8 of values of order one, twice."""
+    from nanoserve_amd.kernels.paged_attention import paged_attention_decode
+    lens = [1, 512, 513, 16 * width - 15, 16 * width, 9000]
+    q, k, v, tables, cl = case(n_heads, n_kv, hd, lens, torch.bfloat16, 5, width=width)
+    args = [t.cuda() for t in (q, k, v, tables, cl)]
+    out = paged_attention_decode(*args, hd ** -0.5)
+    assert (out.cpu().double() - reference(q, k, v, tables, cl, hd ** -0.5)).abs().max().item() <= 1e-2
+    # a row's partitions do not depend on the table width
+    narrow = paged_attention_decode(args[0][:3].contiguous(), args[1], args[2], args[3][:3, :33].contiguous(), args[4][:3], hd ** -0.5)
+    assert torch.equal(narrow, out[:3])
