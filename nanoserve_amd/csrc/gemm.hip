@@ -1022,74 +1022,60 @@ __global__ __launch_bounds__(64) void rms_norm_apply_kernel(const bf16_t* __rest
 // Prefill chunks, mixed steps and speculative verify batches: Y[M, N] = X[M, K] . W[N, K]^T for any M, bf16
 // in, fp32 accumulate, with the STORE (+ bias), SILU, residual-add (RESNORM) and RoPE + K/V-write (ROPE)
 // epilogues of the skinny kernels.
-//   * BM x BN output tiles, NW waves in a WM x (NW / WM) grid, each a (16 FM) x (16 FN) block of
-//     mfma_f32_16x16x32_bf16 tiles. Shapes: 256 x 256 (8 waves of 128 x 64, one workgroup per CU), 256 x 128
-//     (8 of 64 x 64), 128 x 128 (8 of 64 x 32, or 4 of 64 x 64 two per CU) and 128 x 96 (8 of 32 x 48, the
-//     tile plan below). A CU's vector memory path moves about 64 bytes per clock
-//     (L2-resident loads into LDS or VGPRs alike); a 256 x 256 tile asks 7.8 bytes per kFLOP of it, half of
-//     what the MFMA rate allows, a 128 x 128 tile 15.6 -- all of it -- so the plan takes the larger tile
-//     whenever it alone fills the GPU.
-//   * SILU: each wave's FN W-row tiles are FN / 2 gate tiles and the FN / 2 matching up tiles, so a lane
-//     holds gate and up of the same outputs and finishes them in registers.
-//   * K in 32-wide steps through a ring of S LDS stages (BM x 64 bytes of X rows + BN x 64 bytes of W rows
-//     each), filled by buffer DMA (16 bytes per lane, each instruction 16 rows x 64 bytes; rows past M or N
-//     and the empty stages past the slice read zeros through the buffer bounds, with no memory access). Each
-//     64-byte row keeps its four 16-byte chunks XOR-swizzled by (row / 2) & 3, so the 16-lane fragment reads
-//     are free of bank conflicts.
-//   * Software pipeline, one barrier per step: step q waits for the wave's own DMA of stage q + 1 (vmcnt)
-//     and meets the other waves at the barrier (which also retires the fragment reads of step q, freeing
-//     stage q's slot), then issues the MFMAs of step q row by row with, between them, the DMA of stage
-//     q + S into the freed slot and the fragment reads of step q + 1: A fragment i right after row i is
-//     issued (an MFMA reads its sources at issue), the W fragments into the second of two sets. Fragment
-//     reads are inline asm, so the compiler does not drain the DMA ring before them; the barrier's
-//     lgkmcnt(0) is their wait.
-//   * Workgroups map XCD-contiguously: XCD x runs a contiguous run of tiles (same W rows, successive X
-//     rows), which share its L2.
-//   * Few tiles, or long K with fewer tiles than CUs: K is cut into `splits` slices; each publishes its fp32
-//     tile to the workspace (agent-scope stores, a per-tile arrival counter in the fixed counter region) and
-//     the last to arrive sums the slices in slice order -- deterministic -- and runs the epilogue.
-//   * Epilogues: STORE passes the fp32 tile through LDS in 64-row passes (RESNORM adds the residual's
-//     pieces, ROPE rotates a head's low and high dims together); SILU stages only the bf16 outputs (one
-//     pass). All threads then write row-contiguous 16-byte pieces. Roundings to bf16 use the hardware
-//     conversion (round to nearest even); the SiLU is g * rcp(1 + exp2(-g log2 e)) on the transcendental
-//     unit (within 2 ulp of fp32 division before the bf16 rounding).
-constexpr int TG_BK = 32;
-constexpr int TG_CROWS = 64;                  // output rows per STORE epilogue pass
-constexpr int TG_MAX_SPLITS = 16;            // K slices at most
-constexpr int TG_PLAN_SPLITS = 6;             // K slices the plan chooses at most
+//   * BM x BN output tiles, 8 waves in a WM x (8 / WM) grid, each a (16 FM) x (16 FN) block of
+//     mfma_f32_16x16x32_bf16 tiles: 256 x 256 (waves of 128 x 64), 192 x 256 (96 x 64), 128 x 256 and 256 x 128
+//     (64 x 64), 128 x 128 (32 x 64) and 128 x 96 (32 x 48). What a CU does per 64 k of a 256 x 256 tile: 2048
+//     cycles of products per SIMD, 64 KB of copies into LDS and 192 KB of fragment reads out of it (about 1300 and
+//     1500 cycles), so the loop runs at the products' rate only if all three overlap, and smaller tiles are bound by
+//     the LDS reads and copies. The plan below weighs the tiles by their measured times.
+//   * K in slabs of 64 through a ring of S LDS slots (BM + BN rows of 128 bytes each), filled by buffer DMA (16
+//     bytes per lane, each instruction 8 rows x 128 bytes, so whole lines; rows past M or N and slabs past the slice
+//     read zeros through the buffer bounds, with no memory access). A row keeps its eight 16-byte chunks XOR-swizzled
+//     by the row, so the 16-lane fragment reads are free of bank conflicts.
+//   * The two waves of a SIMD work in opposite phases: one multiplies while the other reads its next fragments. With
+//     all waves in step the products of both queued behind each other's reads: 1.62 us per 64 k of 256 x 256 tiles
+//     against 1.38 now, 0.95 against 0.80 for 256 x 128.
+//   * Workgroups map XCD-contiguously: XCD x runs a contiguous run of tiles (at most 7 row tiles of successive column
+//     tiles), which share its L2.
+//   * Long K with fewer tiles than CUs: K is cut into `splits` slices; each publishes its fp32 tile to the workspace
+//     (16-byte coherent stores, a per-tile arrival counter in the fixed counter region); the last to arrive loads the
+//     other slices' tiles and adds them and its own accumulators in slice order -- deterministic -- and runs the
+//     epilogue.
+//   * The products are taken as W . X^T, so a lane holds 4 consecutive outputs of one row per tile, and the W rows are
+//     dealt to the tiles (tg_wrow) such that two tiles give it 8: the epilogues run on the accumulators and write 16
+//     bytes per lane, with no LDS and no barrier. SILU and ROPE deal a wave block the gate and up rows (the low and
+//     high dims of a head) of the same outputs. Roundings to bf16 use the hardware conversion (round to nearest even);
+//     the SiLU is g * rcp(1 + exp2(-g log2 e)) on the transcendental unit (within 2 ulp of fp32 division before the
+//     bf16 rounding).
+// Measured, the launch alone: 1553 rows of 1.5B-shape projections: gate/up 100 -> 92 us, down 76 -> 57, O 18.9 -> 16.1,
+// QKV 25.4 -> 24.6; 3551 rows of 0.5B shapes 88 -> 72, 59 -> 41, 14.3 -> 13.1, 17.5 -> 16.1; 4096 rows of 3B shapes
+// 358 -> 305, 273 -> 168, 48 -> 37, 71 -> 51; 512 rows of 1.5B shapes 48 -> 34, 37 -> 26, 16.6 -> 14.6.
+constexpr int TG_BK = 64;
+constexpr int TG_MAX_SPLITS = 6;             // K slices at most
 constexpr int TG_RSRC3 = 0x00020000;          // buffer resource word 3: raw (untyped) 32-bit accesses
 
-// NW waves in a WM x (NW / WM) grid (wave w at m-block w % WM, n-block w / WM), each a (16 FM) x (16 FN) block.
-template <int FM, int FN, int NW_, int WM_ = 2>
+// 8 waves in a WM x (8 / WM) grid (wave w at m-block w % WM, n-block w / WM), each a (16 FM) x (16 FN) block; one
+// workgroup per CU. K is stepped through in slabs of TG_BK.
+template <int FM, int FN, int WM_>
 struct TgShape {
-  static constexpr int NW = NW_, NT = 64 * NW, WM = WM_, WNW = NW / WM;   // waves, threads, waves along M / N
+  static constexpr int NW = 8, NT = 64 * NW, WM = WM_, WNW = NW / WM;    // waves, threads, waves along M / N
   static constexpr int BM = 16 * FM * WM, BN = 16 * FN * WNW;            // X rows, W rows of a tile
-  static constexpr int WG_PER_CU = NW == 8 ? 1 : 2;
-  static constexpr int S = 4;                                 // ring stages
-  static constexpr int AROWS = BM * TG_BK * 2;                // bytes of the X rows of a stage
+  static constexpr int HV = FM >= 6 ? 2 : 1;                  // phases of a slab: halves of the tall wave blocks' rows
+  static constexpr int S = HV == 2 ? 2 : FM * FN >= 16 ? 3 : FM * FN >= 8 ? 4 : 5;   // slabs the LDS ring holds
+  static constexpr int AROWS = BM * TG_BK * 2;                // bytes of the X rows of a slab
   static constexpr int STAGE = AROWS + BN * TG_BK * 2;
-  static constexpr int CP = BN + 4;                           // floats per row of the staged STORE tile
-  static constexpr int OCP = BN / 2 + 8;                      // bf16 per row of the staged SILU tile
-  static constexpr int CBYTES = TG_CROWS * CP * 4 > BM * OCP * 2 ? TG_CROWS * CP * 4 : BM * OCP * 2;
   static constexpr int PART = BM * BN;                        // floats of one published slice of a tile
-  // DMA instructions of a stage: 16-row groups, GA of X rows then GB of W rows. EVEN: wave w stages X groups
-  // AJ w .. AJ w + AJ - 1 and W groups BJ w .. likewise. Otherwise instruction d of wave w stages group
-  // d NW + w, and the waves left without one issue a no-traffic copy of zeros into a spare 1 KB (DUMMY), so
-  // that every wave counts DMA copies per stage.
-  static constexpr int GA = BM / 16, GB = BN / 16;
-  static constexpr bool EVEN = GA % NW == 0 && GB % NW == 0;
-  static constexpr int AJ = EVEN ? GA / NW : 0, BJ = EVEN ? GB / NW : 0;
-  static constexpr int DMA = EVEN ? AJ + BJ : (GA + GB + NW - 1) / NW;
-  static constexpr int DUMMY = S * STAGE;                     // spare bytes after the ring (not EVEN)
-  static constexpr int RING = EVEN ? S * STAGE : S * STAGE + 1024;
-  static constexpr int LDS0 = RING > CBYTES ? RING : CBYTES;
-  // one workgroup per CU: more than half the CU's 160 KB
-  static constexpr int LDS = WG_PER_CU == 1 && LDS0 <= 80 * 1024 ? 80 * 1024 + 16 : LDS0;
-  static constexpr int MF = FM * FN;                          // MFMAs per wave per step
-  static constexpr int RW = 16 * FM;                          // rows of a wave's block
-  static_assert((RW % TG_CROWS == 0 || TG_CROWS % RW == 0) && (!EVEN || (AJ >= 1 && BJ >= 1)) && DMA <= MF &&
-                    WG_PER_CU * LDS <= 160 * 1024,
-                "tile shape");
+  // DMA instructions of a slab: groups of 8 rows of 128 bytes (1 KB), GA of X rows (of each half) and GB of W rows.
+  // Wave w copies X groups AJ w .. AJ w + AJ - 1 (of each half) and W groups BJ w .. likewise. Where the groups do not
+  // divide evenly, instruction j of wave w takes group j NW + w, and the waves left without one issue a no-traffic
+  // copy of zeros into a spare 1 KB (DUMMY), so that every wave counts the same copies.
+  static constexpr int GA = BM / 8 / HV, GB = BN / 8;
+  static constexpr bool EVEN_A = GA % NW == 0, EVEN_B = GB % NW == 0;
+  static constexpr int AJ = (GA + NW - 1) / NW, BJ = (GB + NW - 1) / NW;
+  static constexpr int DUMMY = S * STAGE;
+  static constexpr int LDS = S * STAGE + (EVEN_A && EVEN_B ? 0 : 1024);
+  static constexpr int MF = FM * FN;                          // MFMAs per wave and 32 k
+  static_assert(LDS + 16 <= 160 * 1024 && GA % WM == 0, "tile shape");
 };
 
 struct TgArgs {
@@ -1098,7 +1084,7 @@ struct TgArgs {
   const bf16_t* bias;
   bf16_t* y;
   int M, N, K;         // N: rows of w (SILU: gate rows then up rows)
-  int tiles_m, tiles_n, splits, kps;   // kps: 32-wide k-steps per slice
+  int tiles_m, tiles_n, splits, kps;   // kps: slabs per slice
   unsigned* cnt;
   float* part;
   const bf16_t* res;   // RESNORM epilogue: y = round(res + round(X W^T)) (the residual sum, no statistics)
@@ -1111,16 +1097,20 @@ struct TgArgs {
   int nh, nkv, hd;
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tg_rsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, int(bytes), TG_RSRC3);
-}
 __device__ __forceinline__ uint32_t tg_lds_addr(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
 }
-// One 16-byte fragment read, no wait: the data is used only after the next barrier, whose lgkmcnt(0)
-// covers it.
-__device__ __forceinline__ void tg_read(uint32_t addr, g_u32x4_t& v) {
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
+// One wave-wide copy of 16 bytes per lane, memory -> LDS (lane i fills lds + 16 i), from the buffer's byte offset
+// voff + soff (out of bounds: zeros, no traffic). Inline asm, so the compiler sees no LDS write in flight and puts
+// no wait for it before the LDS reads of the phase; the vmcnt wait and barrier of the phase loop are the only
+// wait the copies need. M0 holds the wave-uniform LDS address; s_nop 0 is the wait state after M0 is written.
+typedef __attribute__((ext_vector_type(4))) int tg_i32x4_t;
+__device__ __forceinline__ void tg_dma16(tg_i32x4_t rsrc, uint32_t voff, int soff, uint32_t lds) {
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds) : "memory");
+}
+__device__ __forceinline__ tg_i32x4_t tg_words(const void* p, int bytes) {
+  const uint64_t u = reinterpret_cast<uint64_t>(p);
+  return tg_i32x4_t{int(uint32_t(u)), int(uint32_t(u >> 32)), bytes, TG_RSRC3};
 }
 // Workgroup barrier for LDS data (no wait for the wave's outstanding DMA, unlike __syncthreads)
 __device__ __forceinline__ void tg_barrier() {
@@ -1139,166 +1129,79 @@ __host__ __device__ __forceinline__ int tg_xcd_order(int i, int n) {
 }
 // fp32 rounded to bf16 (nearest even, hardware conversion), kept in fp32
 __device__ __forceinline__ float tg_round(float f) { return __uint_as_float(pack_bf16x2(f, 0.f) << 16); }
-// W row staged at row r of a tile's W rows. STORE: BN tn + r. SILU: tile tn covers output columns
-// (BN / 2) tn + [0, BN / 2); wave block c = r / (16 FN) stages its FN / 2 gate tiles, then the matching up tiles.
+// W row staged at row r of a tile's W rows. The products come out with lane l holding rows 4 (l / 16) .. + 3 of a
+// 16-row W tile, so the rows of two neighbouring tiles are dealt such that a lane's 4 + 4 are 8 consecutive outputs
+// (32 outputs per tile pair; a tile without a partner keeps its order, 4 outputs per lane).
+//   STORE, RESNORM: outputs BN tn + [0, BN). SILU: outputs (BN / 2) tn + [0, BN / 2); wave block c = r / (16 FN)
+//   stages its FN / 2 gate tiles, then the matching up tiles. ROPE: wave block c stages 8 FN dims of a head's low
+//   half, then the matching dims of its high half.
+template <int NT>
+__device__ __forceinline__ int tg_deal(int j, int rr) {   // output (of 16 NT) at row rr of tile j
+  if ((NT & 1) != 0 && j == NT - 1) return 16 * j + rr;
+  return 32 * (j >> 1) + 8 * (rr >> 2) + 4 * (j & 1) + (rr & 3);
+}
 template <int EPI, int FN, int BN>
-__device__ __forceinline__ int tg_wrow(int r, int tn, int half) {
-  if constexpr (EPI == EPI_SILU) {
-    const int c = r / (16 * FN), jj = (r / 16) % FN, rr = r % 16;
-    const int oc = (BN / 2) * tn + 8 * FN * c + 16 * (jj % (FN / 2)) + rr;
-    return jj < FN / 2 ? oc : half + oc;
+__device__ __forceinline__ int tg_wrow(const TgArgs& a, int r, int tn) {
+  const int c = r / (16 * FN), jj = (r / 16) % FN, rr = r % 16;
+  if constexpr (EPI == EPI_SILU || EPI == EPI_ROPE) {
+    const int u = jj % (FN / 2), o = tg_deal<FN / 2>(u, rr), lo = (BN / 2) * tn + 8 * FN * c + o;
+    if constexpr (EPI == EPI_SILU) return jj < FN / 2 ? lo : (a.N >> 1) + lo;
+    const int hh = a.hd >> 1, head = lo / hh;   // lo counts the heads' low dims
+    return head * a.hd + (lo - head * hh) + (jj < FN / 2 ? 0 : hh);
   } else {
-    return BN * tn + r;
+    return BN * tn + 16 * FN * c + tg_deal<FN>(jj, rr);
   }
 }
 
-// ROPE epilogue item c of a staged output row (fp32 products, columns n0 .. of the tile): dims d0 .. d0+7 and
-// d0 + hd/2 .. of one head of row gm. The values are rounded as the STORE epilogue stores them (bias added,
-// then bf16), then rotated with the roundings of rope_qkv: lo = round(xl cl) - round(xh sl), hi = round(xh ch)
-// + round(xl sh); value heads pass through. A tile holds whole heads (its width is a multiple of hd).
-__device__ __forceinline__ void tg_rope_item(const TgArgs& a, const float* crow, int gm, int n0, int c) {
-  const int gph = a.hd >> 4, hh = a.hd >> 1;   // 8-dim groups per half head
-  const int ht = c / gph, d0 = 8 * (c - ht * gph), col = ht * a.hd + d0, gn = n0 + col;
-  if (gm >= a.M || gn >= a.N) return;
-  const int head = gn / a.hd;
-  float xl[8], xh[8], lo[8], hi[8];
+// V bf16 values as raw bits, and as floats
+template <int V>
+using tg_raw_t = unsigned int __attribute__((ext_vector_type(V / 2)));
+template <int V>
+__device__ __forceinline__ void tg_unpack(const tg_raw_t<V>& u, float (&v)[V]) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    xl[e] = crow[col + e];
-    xh[e] = crow[col + hh + e];
-  }
-  if (a.bias != nullptr) {
-    float bl[8], bh[8];
-    load_bf16x8(a.bias + gn, bl);
-    load_bf16x8(a.bias + gn + hh, bh);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      xl[e] += bl[e];
-      xh[e] += bh[e];
-    }
-  }
-  if (head < a.nh + a.nkv) {
-    float cl[8], ch[8], sl[8], sh[8];
-    const bf16_t* cr = a.cosb + int64_t(gm) * a.hd + d0;
-    const bf16_t* sr = a.sinb + int64_t(gm) * a.hd + d0;
-    load_bf16x8(cr, cl);
-    load_bf16x8(cr + hh, ch);
-    load_bf16x8(sr, sl);
-    load_bf16x8(sr + hh, sh);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float l = tg_round(xl[e]), h = tg_round(xh[e]);
-      lo[e] = tg_round(l * cl[e]) - tg_round(h * sl[e]);
-      hi[e] = tg_round(h * ch[e]) + tg_round(l * sh[e]);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      lo[e] = xl[e];
-      hi[e] = xh[e];
-    }
-  }
-  bf16_t* dst;
-  bf16_t* cdst = nullptr;
-  if (head < a.nh) {
-    dst = a.q + (int64_t(gm) * a.nh + head) * a.hd;
-  } else if (head < a.nh + a.nkv) {
-    const int kh = head - a.nh;
-    dst = a.k + (int64_t(gm) * a.nkv + kh) * a.hd;
-    if (a.kc != nullptr) cdst = a.kc + (a.slots[gm] * a.nkv + kh) * a.hd;
-  } else {
-    const int vh = head - a.nh - a.nkv;
-    dst = a.v + (int64_t(gm) * a.nkv + vh) * a.hd;
-    if (a.vc != nullptr) cdst = a.vc + (a.slots[gm] * a.nkv + vh) * a.hd;
-  }
-  store_bf16x8(dst + d0, lo);
-  store_bf16x8(dst + d0 + hh, hi);
-  if (cdst != nullptr) {
-    store_bf16x8(cdst + d0, lo);
-    store_bf16x8(cdst + d0 + hh, hi);
+  for (int e = 0; e < V / 2; ++e) {
+    v[2 * e] = __uint_as_float(u[e] << 16);
+    v[2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
   }
 }
+template <int V>
+__device__ __forceinline__ tg_raw_t<V> tg_pack(const float (&v)[V]) {
+  tg_raw_t<V> u;
+#pragma unroll
+  for (int e = 0; e < V / 2; ++e) u[e] = pack_bf16x2(v[2 * e], v[2 * e + 1]);
+  return u;
+}
+// Keeps a computed value (and the loads behind it) in front of the stores that follow: left alone, the compiler
+// sinks loads into the row-bounds branch of their item, which chains the items' latencies.
+template <int V>
+__device__ __forceinline__ void tg_pin(tg_raw_t<V>& u) {
+#pragma unroll
+  for (int e = 0; e < V / 2; ++e) asm volatile("" : "+v"(u[e]));
+}
 
-template <int EPI, int FM, int FN, int NW, int WM>
-__global__ __launch_bounds__((TgShape<FM, FN, NW, WM>::NT), (TgShape<FM, FN, NW, WM>::WG_PER_CU)) void tiled_gemm_kernel(
-    TgArgs a) {
-  using SH = TgShape<FM, FN, NW, WM>;
-  static_assert(EPI != EPI_SILU || (WM == 2 && FN % 4 == 0), "the SiLU epilogue pairs gate and up tiles of a 2-row wave grid");
-  constexpr int BM = SH::BM, BN = SH::BN, NT = SH::NT, S = SH::S;
+template <int EPI, int FM, int FN, int WM>
+__global__ __launch_bounds__((TgShape<FM, FN, WM>::NT), 1) void tiled_gemm_kernel(TgArgs a) {
+  using SH = TgShape<FM, FN, WM>;
+  static_assert((EPI != EPI_SILU && EPI != EPI_ROPE) || FN % 2 == 0, "these epilogues pair the tiles of a wave block");
+  constexpr int BM = SH::BM, BN = SH::BN, NT = SH::NT, NW = SH::NW, S = SH::S;
   __shared__ __align__(16) unsigned char lds[SH::LDS];
   __shared__ unsigned s_last;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const int tiles = a.tiles_m * a.tiles_n, grid = tiles * a.splits;
   const int bid = tg_xcd_order(int(blockIdx.x), grid);
   const int split = bid / tiles, t = bid - split * tiles;
-  const int tm = t % a.tiles_m, tn = t / a.tiles_m;
+  // an XCD's run of tiles covers at most 7 row tiles at a time (X rows read by as many column tiles as W rows are by
+  // row tiles: 4096 x 4096 x 4096 104 -> 99 us)
+  const int t_gs = (a.tiles_m + (a.tiles_m + 6) / 7 - 1) / ((a.tiles_m + 6) / 7), t_g = t / (t_gs * a.tiles_n);
+  const int t_gm = min(t_gs, a.tiles_m - t_g * t_gs), t_in = t - t_g * t_gs * a.tiles_n;
+  const int tm = t_g * t_gs + t_in % t_gm, tn = t_in / t_gm;
   const int m0 = tm * BM;
   const int K = a.K, M = a.M, N = a.N, half = N >> 1;
-  const int kb = split * a.kps, nk = min(a.kps, K / TG_BK - kb);
+  const int k0 = split * a.kps * TG_BK, klen = min(a.kps * TG_BK, K - k0);   // the slice
 
-  // DMA lanes: X instruction j of wave w stages rows 16 (AJ w + j) + l / 4, W instruction j rows
-  // 16 (BJ w + j) + l / 4; slot l % 4 of a row holds chunk (l % 4) ^ ((row / 2) & 3). Row offsets go in the
-  // per-lane offset, so rows past M / N fail the bounds.
-  constexpr int AJ = SH::AJ, BJ = SH::BJ, GA = SH::GA, GB = SH::GB;
-  uint32_t voa[AJ > 0 ? AJ : 1], vob[BJ > 0 ? BJ : 1], vo[SH::DMA];
+  constexpr int AJ = SH::AJ, BJ = SH::BJ;
   const int wu = __builtin_amdgcn_readfirstlane(w);   // the wave index as a scalar (uniform branches)
-  if constexpr (SH::EVEN) {
-#pragma unroll
-    for (int j = 0; j < AJ; ++j) {
-      const int r = 16 * (AJ * w + j) + (l >> 2), c = (l & 3) ^ ((r >> 1) & 3);
-      voa[j] = (uint32_t(m0 + r) * uint32_t(K) + uint32_t(8 * c)) * 2u;
-    }
-#pragma unroll
-    for (int j = 0; j < BJ; ++j) {
-      const int r = 16 * (BJ * w + j) + (l >> 2), c = (l & 3) ^ ((r >> 1) & 3);
-      vob[j] = (uint32_t(tg_wrow<EPI, FN, BN>(r, tn, half)) * uint32_t(K) + uint32_t(8 * c)) * 2u;
-    }
-  } else {
-#pragma unroll
-    for (int d = 0; d < SH::DMA; ++d) {
-      const int gx = d * NW + wu, gw = gx - GA;
-      const int r = 16 * (gx < GA ? gx : gw) + (l >> 2), c = (l & 3) ^ ((r >> 1) & 3);
-      const uint32_t row = gx < GA ? uint32_t(m0 + r) : gw < GB ? uint32_t(tg_wrow<EPI, FN, BN>(r, tn, half)) : 0u;
-      vo[d] = (row * uint32_t(K) + uint32_t(8 * c)) * 2u;
-    }
-  }
-  const __amdgpu_buffer_rsrc_t xr = tg_rsrc(a.x, uint32_t(M) * uint32_t(K) * 2u), xnone = tg_rsrc(a.x, 0u);
-  const __amdgpu_buffer_rsrc_t wr = tg_rsrc(a.w, uint32_t(N) * uint32_t(K) * 2u), wnone = tg_rsrc(a.w, 0u);
-  // DMA instruction d (X rows for d < AJ, then W rows) of stage q of the slice (past nk: zeros, no traffic)
-  auto dma = [&](int q, int d) __attribute__((always_inline)) {
-    const bool live = q < nk;
-    const int soff = __builtin_amdgcn_readfirstlane(live ? (kb + q) * TG_BK * 2 : 0);   // uniform: an SGPR
-    unsigned char* st = lds + (q % S) * SH::STAGE;
-    if constexpr (!SH::EVEN) {
-      const int gx = d * NW + wu, gw = gx - GA;
-      if (gx < GA)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? xr : xnone,
-                                                 (__attribute__((address_space(3))) void*)(st + 16 * gx * 64), 16,
-                                                 int(vo[d]), soff, 0, 0);
-      else if (gw < GB)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            live ? wr : wnone, (__attribute__((address_space(3))) void*)(st + SH::AROWS + 16 * gw * 64), 16,
-            int(vo[d]), soff, 0, 0);
-      else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xnone, (__attribute__((address_space(3))) void*)(lds + SH::DUMMY),
-                                                 16, 0, 0, 0, 0);
-    } else if (d < AJ) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? xr : xnone,
-                                               (__attribute__((address_space(3))) void*)(st + 16 * (AJ * w + d) * 64),
-                                               16, int(voa[d]), soff, 0, 0);
-    } else {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          live ? wr : wnone, (__attribute__((address_space(3))) void*)(st + SH::AROWS + 16 * (BJ * w + d - AJ) * 64), 16,
-          int(vob[d - AJ]), soff, 0, 0);
-    }
-  };
-
-  // fragment offsets within a stage: lane -> row l % 16 of the 16-row tile, 16-byte chunk l / 16; the swizzle
-  // of rows 16 i + l % 16 does not depend on i, so fragment i sits 1024 i bytes further
   const int wm = w % WM, wn = w / WM;
-  const int ra = 16 * FM * wm + (l & 15), rb = 16 * FN * wn + (l & 15);
-  const uint32_t foa = uint32_t(ra * 64 + 16 * ((l >> 4) ^ ((ra >> 1) & 3)));
-  const uint32_t fob = uint32_t(SH::AROWS + rb * 64 + 16 * ((l >> 4) ^ ((rb >> 1) & 3)));
   g_float4_t acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -1306,75 +1209,196 @@ __global__ __launch_bounds__((TgShape<FM, FN, NW, WM>::NT), (TgShape<FM, FN, NW,
     for (int j = 0; j < FN; ++j) acc[i][j] = g_float4_t{0.f, 0.f, 0.f, 0.f};
   const uint32_t lds0 = tg_lds_addr(lds);
 
-  // RESNORM: the thread's residual pieces for the epilogue's items (item k of 64-row pass p: it = tid + k NT,
-  // row it / (BN / 8), 8 columns it % (BN / 8)), loaded before the K loop so their latency hides under it,
-  // when they fit in 8 registers of 16 bytes (else each item loads its own). Addresses are clamped into the
-  // residual, so the loads are unconditional; pieces past M or N are never used.
-  constexpr int RIPR = BN / 8, RIPT = (TG_CROWS * RIPR + NT - 1) / NT;   // items per thread and pass, at most
-  static_assert(TG_CROWS * RIPR % 64 == 0 && TG_CROWS * (BN / 16) % 64 == 0, "epilogue items: whole waves");
-  constexpr int RPRE = EPI == EPI_RESNORM && BM / TG_CROWS * RIPT <= 8 ? BM / TG_CROWS * RIPT : 0;
-  g_u32x4_t rres[RPRE > 0 ? RPRE : 1];
-  if constexpr (RPRE > 0) {
+  // Outputs: lane l holds, of X tile i and the W tile pair p, row 16 i + l % 16 of the wave's block, columns 32 p +
+  // 8 (l / 16) .. + 7 (a last tile without a partner: 4 columns).
+  constexpr int FP = FN / 2;
+  const int row0 = m0 + 16 * FM * wm + (l & 15), col0 = BN * tn + 16 * FN * wn, cl8 = 8 * (l >> 4);
+  // RESNORM: the lane's residual pieces, loaded before the K loop so their latency hides under it, when they fit in
+  // 8 registers of 16 bytes (else each is loaded where it is added). Addresses are clamped into the residual, so the
+  // loads are unconditional; pieces past M or N are never used.
+  constexpr bool RPRE = EPI == EPI_RESNORM && FN % 2 == 0 && FM * FP <= 8;
+  g_u32x4_t rres[RPRE ? FM * FP : 1];
+  if constexpr (RPRE) {
 #pragma unroll
-    for (int u = 0; u < RPRE; ++u) {
-      const int it = tid + (u % RIPT) * NT;
-      const int gm = min(m0 + TG_CROWS * (u / RIPT) + it / RIPR, M - 1), gn = min(BN * tn + 8 * (it % RIPR), N - 8);
+    for (int u = 0; u < FM * FP; ++u) {
+      const int gm = min(row0 + 16 * (u / FP), M - 1), gn = min(col0 + 32 * (u % FP) + cl8, N - 8);
       rres[u] = *reinterpret_cast<const g_u32x4_t*>(a.res + int64_t(gm) * N + gn);
     }
   }
 
-  // Step q: the MFMAs of step q, row by row, from A and Bc; between them the DMA of stage q + S, and the
-  // reads of step q + 1: A[i] as soon as row i is issued, Bn spread over the step.
-  g_u32x4_t A[FM], B0[FN], B1[FN];
-  auto step = [&](int q, g_u32x4_t (&Bc)[FN], g_u32x4_t (&Bn)[FN]) __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(tg_vmcnt(SH::DMA * (S - 2)));   // this wave's loads of stage q + 1 are done
-    tg_barrier();   // ... and every wave's; every read of step q has landed, so stage q's slot is free
-    __builtin_amdgcn_sched_barrier(0);
-    const uint32_t sn = lds0 + uint32_t(((q + 1) % S) * SH::STAGE);
-    constexpr int EVERY = SH::MF / FN;
-#pragma unroll
-    for (int u = 0; u < SH::MF; ++u) {
-      const int i = u / FN, j = u % FN;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(g_bf16x8_t, A[i]),
-                                                         __builtin_bit_cast(g_bf16x8_t, Bc[j]), acc[i][j], 0, 0, 0);
-      if (u < SH::DMA) dma(q + S, u);
-      if (j == FN - 1) tg_read(sn + foa + 1024u * i, A[i]);
-      if (u % EVERY == EVERY / 2) tg_read(sn + fob + 1024u * (u / EVERY), Bn[u / EVERY]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  // Two wave groups in opposite phases: waves 0..3 and 4..7 sit on the same four SIMDs, and while one group
+  // multiplies, the other reads its fragments and waits for them. Each group alternates a
+  // memory half and a multiply half, a barrier after each; group 1 starts half a phase late. A slot's rows are
+  // overwritten by copies issued after the half that used them: both groups have by then
+  // passed the barrier that follows their reads (and the wait for them). Copies are waited for by the wave that
+  // issued them before the barrier that precedes group 0's reads of them: group 0 at the end of its multiply
+  // half, group 1, half a phase later in the loop, at the end of its memory half. The copies are issued between the
+  // products of the multiply half, except for the tallest wave blocks, which issue them in the memory half (a slot's
+  // rows are then free half a phase earlier). Per 64-wide slab, one tile per CU, products at 16 of 16 row tiles:
+  // 256 x 128 tiles 0.97 us with the copies in the memory half, 0.90 between the products; 128 x 128 0.59, 0.51;
+  // 128 x 96 0.53, 0.41; 256 x 256 1.48, 1.55.
+  constexpr int HV = SH::HV, FH = FM / HV, BK = TG_BK;
+  const bool g1 = wu >= NW / 2;
+  const int n_sl = (klen + BK - 1) / BK;
+  const bool odd = (klen & (BK - 1)) != 0;   // the last slab holds 32 k: its other chunks read zeros
+  const uint32_t xbytes = uint32_t(M) * uint32_t(K) * 2u, wbytes = uint32_t(N) * uint32_t(K) * 2u;
+  const tg_i32x4_t xw = tg_words(a.x, int(xbytes)), ww = tg_words(a.w, int(wbytes));
+  // DMA lanes: a group's lane l fills slot l % 8 of row l / 8, which holds the row's 16-byte chunk
+  // (l % 8) ^ key(row), key(row) = (row & 7) ^ ((row >> 3) & 1): the 16 rows of a fragment read then touch 16
+  // different 16-byte columns of the 256 bytes that their row pairs span. Whole 128-byte lines per row: with
+  // 64-byte pieces (32 k per stage) the copies, not the products, bounded the loop. Row offsets go in the
+  // per-lane offset, so rows past M / N fail the bounds.
+  uint32_t voa[HV][AJ], vob[BJ];
+  auto chunk = [&](int r) __attribute__((always_inline)) { return (l & 7) ^ (r & 7) ^ ((r >> 3) & 1); };
+  auto agroup = [&](int j, int wave) __attribute__((always_inline)) { return SH::EVEN_A ? AJ * wave + j : j * NW + wave; };
+  auto arow = [&](int h, int j, int wave) __attribute__((always_inline)) {   // first X row of copy j of half h
+    const int gi = agroup(j, wave), per = SH::GA / WM;   // per: groups of a wave block's half
+    return HV == 1 ? 8 * gi : 16 * FM * (gi / per) + 16 * FH * h + 8 * (gi % per);
   };
-
+  auto bgroup = [&](int j, int wave) __attribute__((always_inline)) { return SH::EVEN_B ? BJ * wave + j : j * NW + wave; };
+  const int lr = l >> 3;
 #pragma unroll
-  for (int q = 0; q < S; ++q)
+  for (int h = 0; h < HV; ++h)
 #pragma unroll
-    for (int d = 0; d < SH::DMA; ++d) dma(q, d);
-  __builtin_amdgcn_s_waitcnt(tg_vmcnt(SH::DMA * (S - 1)));   // stage 0
-  tg_barrier();
+    for (int j = 0; j < AJ; ++j) {
+      const int r = arow(h, j, w) + lr;
+      voa[h][j] = SH::EVEN_A || agroup(j, w) < SH::GA ? (uint32_t(m0 + r) * uint32_t(K) + uint32_t(8 * chunk(r))) * 2u : xbytes;
+    }
 #pragma unroll
-  for (int i = 0; i < FM; ++i) tg_read(lds0 + foa + 1024u * i, A[i]);
-#pragma unroll
-  for (int j = 0; j < FN; ++j) tg_read(lds0 + fob + 1024u * j, B0[j]);
-  for (int q = 0;; q += 2) {
-    step(q, B0, B1);
-    if (q + 1 >= nk) break;
-    step(q + 1, B1, B0);
-    if (q + 2 >= nk) break;
+  for (int j = 0; j < BJ; ++j) {
+    const int r = 8 * bgroup(j, w) + lr;
+    vob[j] = SH::EVEN_B || r < BN ? (uint32_t(tg_wrow<EPI, FN, BN>(a, r, tn)) * uint32_t(K) + uint32_t(8 * chunk(r))) * 2u : wbytes;
   }
+  // one copy of slab q; past the slice: zeros, no traffic
+  auto put = [&](tg_i32x4_t r, uint32_t vo, uint32_t none, int row, int q, uint32_t dst) __attribute__((always_inline)) {
+    if (q >= n_sl) r[2] = 0;
+    if (odd && q == n_sl - 1) vo = chunk(row + lr) >= 4 ? none : vo;
+    tg_dma16(r, vo, q < n_sl ? (k0 + q * BK) * 2 : 0, dst);
+  };
+  auto copy_x = [&](int h, int j, int q, int slot) __attribute__((always_inline)) {
+    const int row = arow(h, j, wu);
+    put(xw, voa[h][j], xbytes, row, q,
+        lds0 + uint32_t(SH::EVEN_A || agroup(j, wu) < SH::GA ? slot * SH::STAGE + row * 128 : SH::DUMMY));
+  };
+  auto copy_w = [&](int j, int q, int slot) __attribute__((always_inline)) {
+    const int g = bgroup(j, wu);
+    put(ww, vob[j], wbytes, 8 * g, q,
+        lds0 + uint32_t(SH::EVEN_B || g < SH::GB ? slot * SH::STAGE + SH::AROWS + g * 1024 : SH::DUMMY));
+  };
+  auto copy_xw = [&](int h, int u, int q, int slot) __attribute__((always_inline)) {   // X copies of half h, then W's
+    if (u < AJ) copy_x(h, u, q, slot); else copy_w(u - AJ, q, slot);
+  };
+  // fragment reads: row l % 16 of a 16-row tile, chunk 4 s + l / 16 of k-step s
+  const int rr = l & 15, kx = (rr & 7) ^ (rr >> 3);
+  uint32_t foa[2], fob[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const uint32_t c = 16u * uint32_t((4 * s + (l >> 4)) ^ kx);
+    foa[s] = uint32_t((16 * FM * wm + rr) * 128) + c;
+    fob[s] = uint32_t(SH::AROWS + (16 * FN * wn + rr) * 128) + c;
+  }
+  g_u32x4_t A[2][FH], B[2][FN];
+  auto read_x = [&](int h, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < FH; ++i)
+        A[s][i] = *reinterpret_cast<const g_u32x4_t*>(lds + slot * SH::STAGE + foa[s] + 2048 * (FH * h + i));
+  };
+  auto read_w = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) B[s][j] = *reinterpret_cast<const g_u32x4_t*>(lds + slot * SH::STAGE + fob[s] + 2048 * j);
+  };
+  // The end of a memory half, then the multiply half of rows h with the wave's n copies (copy(u), u < n) spread over
+  // it. left0 / left1: copies that may stay outstanding at the end of group 0's multiply half / group 1's memory half.
+  auto multiply = [&](auto h_c, auto n_c, auto left0, auto left1, auto&& copy) __attribute__((always_inline)) {
+    constexpr int h = decltype(h_c)::value, n = decltype(n_c)::value, MFS = 2 * FH * FN, EVERY = n > 0 ? MFS / n : MFS;
+    if (g1) __builtin_amdgcn_s_waitcnt(tg_vmcnt(decltype(left1)::value));
+    tg_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int u = 0; u < MFS; ++u) {
+      const int s = u / (FH * FN), i = u / FN % FH, j = u % FN;
+      acc[FH * h + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(g_bf16x8_t, B[s][j]), __builtin_bit_cast(g_bf16x8_t, A[s][i]), acc[FH * h + i][j], 0, 0, 0);
+      if (u % EVERY == EVERY / 2 && u / EVERY < n) {
+        __builtin_amdgcn_sched_barrier(0);
+        copy(u / EVERY);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!g1) __builtin_amdgcn_s_waitcnt(tg_vmcnt(decltype(left0)::value));
+    tg_barrier();
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 0> C0{};
+  if constexpr (HV == 1) {
+    constexpr int R = AJ + BJ;
+#pragma unroll
+    for (int q = 0; q < S - 1; ++q)
+#pragma unroll
+      for (int u = 0; u < R; ++u) copy_xw(0, u, q, q);
+    __builtin_amdgcn_s_waitcnt(tg_vmcnt(R * (S - 2)));   // slab 0
+    tg_barrier();
+    if (g1) tg_barrier();
+    for (int q = 0, slot = 0; q < n_sl; ++q, slot = slot + 1 == S ? 0 : slot + 1) {
+      read_w(slot);
+      read_x(0, slot);
+      __builtin_amdgcn_sched_barrier(0);
+      const int free_slot = slot == 0 ? S - 1 : slot - 1;
+      multiply(C0, integral_constant<int, R>{}, integral_constant<int, R * (S - 2)>{}, integral_constant<int, R * (S - 3)>{},
+               [&](int u) __attribute__((always_inline)) { copy_xw(0, u, q + S - 1, free_slot); });
+    }
+  } else {
+    // two slots; the rows of a slot are refilled half by half as soon as they have been read: half 1 of slab q + 1 in
+    // the first phase of slab q, W and the X rows of half 0 of slab q + 2 in the second
+    constexpr integral_constant<int, 1> C1{};
+    constexpr int R = AJ + BJ;
+    constexpr integral_constant<int, R + AJ> both{};
+    auto none = [](int) {};
+#pragma unroll
+    for (int u = 0; u < R; ++u) copy_xw(0, u, 0, 0);
+#pragma unroll
+    for (int u = 0; u < AJ; ++u) copy_x(1, u, 0, 0);
+#pragma unroll
+    for (int u = 0; u < R; ++u) copy_xw(0, u, 1, 1);
+    __builtin_amdgcn_s_waitcnt(tg_vmcnt(both));   // half 0 of slab 0
+    tg_barrier();
+    if (g1) tg_barrier();
+    for (int q = 0; q < n_sl; ++q) {
+      const int slot = q & 1;
+      read_w(slot);
+      read_x(0, slot);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < AJ; ++u) copy_x(1, u, q + 1, slot ^ 1);
+      multiply(C0, C0, both, both, none);
+      read_x(1, slot);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < R; ++u) copy_xw(0, u, q + 2, slot);
+      multiply(C1, C0, both, both, none);
+    }
+  }
+  if (!g1) tg_barrier();
   __builtin_amdgcn_s_waitcnt(tg_vmcnt(0));
   tg_barrier();
 
   // ---- K slices: publish, count, and the last slice sums them in slice order
-  if (a.splits > 1) {
-    float* mine = a.part + (int64_t(t) * a.splits + split) * SH::PART;
+  constexpr bool SLICES = EPI != EPI_SILU && SH::MF <= 16;   // what the plan may slice
+  if constexpr (SLICES) if (a.splits > 1) {
+    constexpr int SC1 = 16;   // cache policy sc1: device-coherent, past the XCD's L2
+    const __amdgpu_buffer_rsrc_t parts = __builtin_amdgcn_make_buffer_rsrc(
+        a.part + int64_t(t) * a.splits * SH::PART, (short)0, a.splits * SH::PART * 4, TG_RSRC3);
+    auto at = [&](int slice, int f) __attribute__((always_inline)) { return (slice * SH::PART + (f * NT + tid) * 4) * 4; };
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const g_float4_t v = acc[i][j];
-        publish_store16(mine + (int64_t(i * FN + j) * NT + tid) * 4,
-                        pub_u32x4_t{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
-                                    __float_as_uint(v[3])});
-      }
+    for (int f = 0; f < SH::MF; ++f)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(pub_u32x4_t, acc[f / FN][f % FN]), parts, at(split, f), 0, SC1);
     publish_complete();
     __syncthreads();
     if (tid == 0) {
@@ -1386,140 +1410,209 @@ __global__ __launch_bounds__((TgShape<FM, FN, NW, WM>::NT), (TgShape<FM, FN, NW,
     __syncthreads();
     if (s_last == 0u) return;
     acquire_published();
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = g_float4_t{0.f, 0.f, 0.f, 0.f};
-    const float* base = a.part + int64_t(t) * a.splits * SH::PART;
-    constexpr int FB = SH::MF < 16 ? SH::MF : 16;   // partial fragments per round trip
-    for (int s = 0; s < a.splits; ++s) {
+    // the other slices' partials, as many fragments of all of them per round trip as registers hold, and this one's own
+    // accumulators, summed in slice order
+    constexpr int FLIGHT = RPRE ? 24 : 32;   // fragments in flight
+    auto merge = [&](auto n_c) __attribute__((always_inline)) {
+      constexpr int SP = decltype(n_c)::value, TRIPS = (SH::MF * (SP - 1) + FLIGHT - 1) / FLIGHT, FB = (SH::MF + TRIPS - 1) / TRIPS;
 #pragma unroll
       for (int f0 = 0; f0 < SH::MF; f0 += FB) {
-        pub_u32x4_t v[FB];
+        pub_u32x4_t v[SP - 1][FB];
+#pragma unroll
+        for (int x = 0; x < SP - 1; ++x)
+#pragma unroll
+          for (int e = 0; e < FB; ++e)
+            if (f0 + e < SH::MF)
+              v[x][e] = __builtin_amdgcn_raw_buffer_load_b128(parts, at(x < split ? x : x + 1, f0 + e), 0, SC1);
 #pragma unroll
         for (int e = 0; e < FB; ++e)
-          v[e] = publish_load16(base + int64_t(s) * SH::PART + (int64_t(f0 + e) * NT + tid) * 4);
+          if (f0 + e < SH::MF)
 #pragma unroll
-        for (int e = 0; e < FB; ++e)
+            for (int r = 0; r < 4; ++r) {
+              const float own = acc[(f0 + e) / FN][(f0 + e) % FN][r];
+              float sum = 0.f;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[(f0 + e) / FN][(f0 + e) % FN][r] += __uint_as_float(v[e][r]);
+              for (int x = 0; x < SP; ++x) {   // slice x: v[x] before the own slice, v[x - 1] after it
+                const float lo = x < SP - 1 ? __uint_as_float(v[x < SP - 1 ? x : 0][e][r]) : 0.f;
+                const float hi = x > 0 ? __uint_as_float(v[x > 0 ? x - 1 : 0][e][r]) : 0.f;
+                sum += x < split ? lo : x == split ? own : hi;
+              }
+              acc[(f0 + e) / FN][(f0 + e) % FN][r] = sum;
+            }
       }
+    };
+    switch (a.splits) {
+      case 2: merge(std::integral_constant<int, 2>{}); break;
+      case 3: merge(std::integral_constant<int, 3>{}); break;
+      case 4: merge(std::integral_constant<int, 4>{}); break;
+      case 5: merge(std::integral_constant<int, 5>{}); break;
+      default: merge(std::integral_constant<int, 6>{}); break;   // TG_MAX_SPLITS
     }
   }
 
-  // Lane layout of acc[i][j]: column 16 FN wn + 16 j + l % 16 of the tile, rows 16 FM wm + 16 i + 4 (l / 16) + r.
-  if constexpr (EPI != EPI_SILU) {
-    // the fp32 tile through LDS in passes of 64 rows (pass p: the waves with wm == p / (FM / 4), their
-    // m-tiles 4 (p % (FM / 4)) .. + 3), then items (row m, 8 columns) of 16 bytes (RESNORM: plus the
-    // residual's 8); ROPE: items (row m, 8 dims of a head's low half and the matching 8 of its high half)
-    float* C = reinterpret_cast<float*>(lds);
-    constexpr int CP = SH::CP, PASSES = BM / TG_CROWS, IPR = EPI == EPI_ROPE ? BN / 16 : BN / 8;
+  // ---- epilogues, straight from the accumulators: 16 rows x 64 bytes per store instruction
+  if constexpr (EPI == EPI_SILU || EPI == EPI_ROPE) {
+    // the wave block's FN / 2 gate (low-half) tiles, then the matching up (high-half) ones
+    constexpr int H = FN / 2, V = H % 2 == 0 ? 8 : 4, Q = 8 * FN / (4 * V);   // V outputs per lane, Q groups of them
 #pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-      if constexpr (SH::RW >= TG_CROWS) {   // a wave block spans PW passes
-        constexpr int PW = SH::RW / TG_CROWS;
-        if (wm == p / PW) {
+    for (int p = 0; p < Q; ++p) {
+      const int gn = (BN / 2) * tn + 8 * FN * wn + 4 * V * p + V * (l >> 4);
+      auto pair = [&](int i, float (&lo)[V], float (&hi)[V]) __attribute__((always_inline)) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                C[(16 * i + 4 * (l >> 4) + r) * CP + 16 * FN * wn + 16 * j + (l & 15)] = acc[4 * (p % PW) + i][j][r];
+        for (int e = 0; e < V; ++e) {
+          lo[e] = acc[i][p * (V / 4) + e / 4][e % 4];
+          hi[e] = acc[i][H + p * (V / 4) + e / 4][e % 4];
         }
-      } else {   // a pass holds WPP wave blocks
-        constexpr int WPP = TG_CROWS / SH::RW;
-        if (wm / WPP == p) {
+      };
+      if constexpr (EPI == EPI_ROPE) {
+        // The values are rounded as the STORE epilogue stores them (bias added, then bf16), then rotated with the
+        // roundings of rope_qkv: lo = round(xl cl) - round(xh sl), hi = round(xh ch) + round(xl sh); value heads pass
+        // through. A wave block lies within one head, so everything about the head is scalar.
+        typedef tg_raw_t<V> raw;
+        const int hd = a.hd, hh = hd >> 1;
+        const int g0 = __builtin_amdgcn_readfirstlane((BN / 2) * tn + 8 * FN * wn + 4 * V * p), head = g0 / hh;
+        if (head * hd >= N) continue;
+        const int d = g0 - head * hh + V * (l >> 4);
+        const int kh = head - a.nh, vh = kh - a.nkv;   // >= 0: a key / value head
+        bf16_t* out = kh < 0 ? a.q + head * hd : vh < 0 ? a.k + kh * hd : a.v + vh * hd;
+        bf16_t* cache = kh < 0 || a.kc == nullptr ? nullptr : vh < 0 ? a.kc + kh * hd : a.vc + vh * hd;
+        const int64_t row = int64_t(kh < 0 ? a.nh : a.nkv) * hd;
+        const bf16_t* bp = a.bias != nullptr ? a.bias + head * hd + d : a.w;   // (any readable memory without a bias:
+        const raw rbl = *reinterpret_cast<const raw*>(bp);                     // a load inside a branch is waited for
+        const raw rbh = *reinterpret_cast<const raw*>(bp + (a.bias != nullptr ? hh : 0));   // at the branch's end)
+        constexpr int IB = V == 8 ? 2 : 4;   // items whose operands are in flight together
+        static_assert(FM % IB == 0, "whole batches");
 #pragma unroll
-          for (int i = 0; i < FM; ++i)
+        for (int i0 = 0; i0 < FM; i0 += IB) {
+          raw c0[IB], c1[IB], s0[IB], s1[IB], olo[IB], ohi[IB];
+          int64_t slot[IB];
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
+          for (int i = 0; i < IB; ++i) {
+            const int gm = min(row0 + 16 * (i0 + i), M - 1);
+            const int64_t at = int64_t(gm) * hd + d;
+            c0[i] = *reinterpret_cast<const raw*>(a.cosb + at);
+            c1[i] = *reinterpret_cast<const raw*>(a.cosb + at + hh);
+            s0[i] = *reinterpret_cast<const raw*>(a.sinb + at);
+            s1[i] = *reinterpret_cast<const raw*>(a.sinb + at + hh);
+            slot[i] = *(cache != nullptr ? a.slots + gm : reinterpret_cast<const int64_t*>(a.cosb));
+          }
 #pragma unroll
-              for (int r = 0; r < 4; ++r)
-                C[(SH::RW * (wm % WPP) + 16 * i + 4 * (l >> 4) + r) * CP + 16 * FN * wn + 16 * j + (l & 15)] =
-                    acc[i][j][r];
-        }
-      }
-      tg_barrier();   // LDS only: the global stores of the previous pass need not land first
-      const int mb = m0 + TG_CROWS * p;
-      constexpr int IPT = (TG_CROWS * IPR + NT - 1) / NT;   // items per thread and pass, at most
+          for (int i = 0; i < IB; ++i) {
+            float xl[V], xh[V], bl[V], bh[V], cl[V], ch[V], sl[V], sh[V];
+            pair(i0 + i, xl, xh);
+            tg_unpack<V>(rbl, bl);
+            tg_unpack<V>(rbh, bh);
+            tg_unpack<V>(c0[i], cl);
+            tg_unpack<V>(c1[i], ch);
+            tg_unpack<V>(s0[i], sl);
+            tg_unpack<V>(s1[i], sh);
 #pragma unroll
-      for (int k = 0; k < IPT; ++k) {
-        const int it = tid + k * NT, m = it / IPR, c8 = it % IPR, gm = mb + m, gn = BN * tn + 8 * c8;
-        if (TG_CROWS * IPR % NT != 0 && it >= TG_CROWS * IPR) continue;   // whole waves (checked above)
-        if constexpr (EPI == EPI_ROPE) {
-          tg_rope_item(a, C + m * CP, gm, BN * tn, c8);
-          continue;
-        }
-        if (gm >= M || gn >= N) continue;
-        float v[8];
+            for (int e = 0; e < V; ++e) {
+              const float l = tg_round(xl[e] + (a.bias != nullptr ? bl[e] : 0.f)), h = tg_round(xh[e] + (a.bias != nullptr ? bh[e] : 0.f));
+              xl[e] = vh < 0 ? tg_round(l * cl[e]) - tg_round(h * sl[e]) : l;
+              xh[e] = vh < 0 ? tg_round(h * ch[e]) + tg_round(l * sh[e]) : h;
+            }
+            olo[i] = tg_pack<V>(xl);
+            ohi[i] = tg_pack<V>(xh);
+            tg_pin<V>(olo[i]);
+            tg_pin<V>(ohi[i]);
+          }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = C[m * CP + 8 * c8 + e];
-        if (a.bias != nullptr) {
-          if ((N & 7) == 0) {
-            float b[8];
-            load_bf16x8(a.bias + gn, b);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] += b[e];
-          } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] += gn + e < N ? bf16_to_f32(a.bias[gn + e]) : 0.f;
+          for (int i = 0; i < IB; ++i) {
+            const int gm = row0 + 16 * (i0 + i);
+            if (gm >= M) continue;
+            bf16_t* dst = out + int64_t(gm) * row + d;
+            *reinterpret_cast<raw*>(dst) = olo[i];
+            *reinterpret_cast<raw*>(dst + hh) = ohi[i];
+            if (cache != nullptr) {
+              bf16_t* cdst = cache + slot[i] * row + d;   // a key / value row: n_kv heads
+              *reinterpret_cast<raw*>(cdst) = olo[i];
+              *reinterpret_cast<raw*>(cdst + hh) = ohi[i];
+            }
           }
         }
-        if constexpr (EPI == EPI_RESNORM) {   // N % 8 == 0 (checked by the entry point)
-          g_u32x4_t u;
-          if constexpr (RPRE > 0)
-            u = rres[p * IPT + k];
-          else
-            u = *reinterpret_cast<const g_u32x4_t*>(a.res + int64_t(gm) * N + gn);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[2 * e] = __uint_as_float(u[e] << 16) + tg_round(v[2 * e]);
-            v[2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u) + tg_round(v[2 * e + 1]);
-          }
-        }
-        bf16_t* dst = a.y + int64_t(gm) * N + gn;
-        if ((N & 7) == 0) {
-          store_bf16x8(dst, v);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (gn + e < N) dst[e] = f32_to_bf16(v[e]);
-        }
-      }
-      if (p + 1 < PASSES) tg_barrier();
-    }
-  } else {
-    // SILU: gate acc[i][j], up acc[i][j + FN / 2] -> output column 8 FN wn + 16 j + l % 16 of the tile's
-    // BN / 2; the bf16 outputs go through LDS ([BM][OCP]) in one pass, then items (row m, 8 columns)
-    bf16_t* O = reinterpret_cast<bf16_t*>(lds);
-    constexpr int OCP = SH::OCP, IPR = BN / 16;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN / 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float gb = tg_round(acc[i][j][r]), ub = tg_round(acc[i][j + FN / 2][r]);
-          const float sg = gb * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gb * -1.44269504088896341f));
-          O[(16 * FM * wm + 16 * i + 4 * (l >> 4) + r) * OCP + 8 * FN * wn + 16 * j + (l & 15)] =
-              bf16_t(pack_bf16x2(tg_round(sg) * ub, 0.f));
-        }
-    tg_barrier();
-#pragma unroll 2
-    for (int it = tid; it < BM * IPR; it += NT) {
-      const int m = it / IPR, c8 = it % IPR, gm = m0 + m, gn = (BN / 2) * tn + 8 * c8;
-      if (gm >= M || gn >= half) continue;
-      const g_u32x4_t v = *reinterpret_cast<const g_u32x4_t*>(O + m * OCP + 8 * c8);
-      bf16_t* dst = a.y + int64_t(gm) * half + gn;
-      if ((half & 7) == 0) {
-        *reinterpret_cast<g_u32x4_t*>(dst) = v;
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (gn + e < half) dst[e] = bf16_t(v[e >> 1] >> (16 * (e & 1)));
+        for (int i = 0; i < FM; ++i) {
+          // round(round(silu(round(g))) * round(u)), silu(g) = g * rcp(1 + exp2(-g log2 e))
+          const int gm = row0 + 16 * i;
+          float lo[V], hi[V], o[V];
+          pair(i, lo, hi);
+#pragma unroll
+          for (int e = 0; e < V; ++e) {
+            const float gb = tg_round(lo[e]), ub = tg_round(hi[e]);
+            o[e] = tg_round(gb * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gb * -1.44269504088896341f))) * ub;
+          }
+          if (gm < M && gn < half) {
+            bf16_t* dst = a.y + int64_t(gm) * half + gn;
+            if ((half & (V - 1)) == 0) {
+              *reinterpret_cast<tg_raw_t<V>*>(dst) = tg_pack<V>(o);
+            } else {
+#pragma unroll
+              for (int e = 0; e < V; ++e)
+                if (gn + e < half) dst[e] = f32_to_bf16(o[e]);
+            }
+          }
+        }
       }
     }
+  } else {
+    // STORE: round(acc + bias); RESNORM: round(res + round(acc)) (N % 8 == 0, checked by the entry point). Column
+    // group p: the tile pair 2 p, 2 p + 1 (V = 8 columns per lane), or a last tile on its own (V = 4).
+    auto columns = [&](auto v_c, int p) __attribute__((always_inline)) {
+      constexpr int V = decltype(v_c)::value, IB = FM % 4 == 0 ? 4 : FM % 3 == 0 ? 3 : FM;   // IB residual pieces in flight together
+      static_assert(FM % IB == 0, "whole batches");
+      typedef tg_raw_t<V> raw;
+      const int gn = col0 + 32 * p + V * (l >> 4);
+      float b[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) b[e] = 0.f;
+      if (EPI == EPI_STORE && a.bias != nullptr)
+#pragma unroll
+        for (int e = 0; e < V; ++e) b[e] = gn + e < N ? bf16_to_f32(a.bias[gn + e]) : 0.f;
+#pragma unroll
+      for (int i0 = 0; i0 < FM; i0 += IB) {
+        raw res[IB], o[IB];
+        if constexpr (EPI == EPI_RESNORM) {
+#pragma unroll
+          for (int i = 0; i < IB; ++i) {
+            if constexpr (RPRE)
+              res[i] = rres[(i0 + i) * FP + p];
+            else
+              res[i] = *reinterpret_cast<const raw*>(a.res + int64_t(min(row0 + 16 * (i0 + i), M - 1)) * N + min(gn, N - V));
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+          float v[V], r[V];
+#pragma unroll
+          for (int e = 0; e < V; ++e) v[e] = acc[i0 + i][2 * p + e / 4][e % 4] + b[e];
+          if constexpr (EPI == EPI_RESNORM) {
+            tg_unpack<V>(res[i], r);
+#pragma unroll
+            for (int e = 0; e < V; ++e) v[e] = r[e] + tg_round(v[e]);
+          }
+          o[i] = tg_pack<V>(v);
+          if constexpr (EPI == EPI_RESNORM) tg_pin<V>(o[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+          const int gm = row0 + 16 * (i0 + i);
+          if (gm >= M || gn >= N) continue;
+          bf16_t* dst = a.y + int64_t(gm) * N + gn;
+          if ((N & 7) == 0) {
+            *reinterpret_cast<raw*>(dst) = o[i];
+          } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+              if (gn + e < N) dst[e] = bf16_t(o[i][e >> 1] >> (16 * (e & 1)));
+          }
+        }
+      }
+    };
+#pragma unroll
+    for (int p = 0; p < FP; ++p) columns(std::integral_constant<int, 8>{}, p);
+    if constexpr (FN % 2 != 0) columns(std::integral_constant<int, 4>{}, FP);
   }
 }
 
@@ -1724,93 +1817,64 @@ static int bind_xnorm(GemmArgs& a, const float* x_sumsq, const void* x_norm_w, f
 }
 
 // ---- tiled GEMM plan and launch (M > 64)
-enum TgTile { TG_SMALL = 0, TG_BIG = 1, TG_TALL = 2, TG_SMALL8 = 3, TG_N96 = 4 };
+// The tiles a plan chooses from, with their measured cost: ns per 64-wide slab of a launch that fills the CUs (16 x 16
+// tiles, K 512 .. 4096), and the rest of a tile's time (first copies, epilogue, launch). Every shape runs one workgroup
+// per CU, so a launch takes ceil(tiles * slices / 256) rounds of (slabs * slab + fixed).
+struct TgTile {
+  int bm, bn, slab, fixed;
+  bool silu, rope, split;   // epilogues that fit its wave blocks; long K may be sliced
+};
+enum { TG_256x256, TG_192x256, TG_128x256, TG_256x128, TG_128x128, TG_128x96, TG_TILES };
+constexpr TgTile TG_TILE[TG_TILES] = {
+    {256, 256, 1380, 11000, true, true, false},  {192, 256, 1080, 10000, true, true, false},
+    {128, 256, 810, 8500, true, true, false},    {256, 128, 800, 8500, false, true, true},
+    {128, 128, 490, 7000, true, true, true},     {128, 96, 420, 7000, false, false, true},
+};
 struct TgPlan {
-  int shape;   // TgTile: 128 x 128 (4 waves, two per CU), 256 x 256 or 256 x 128 (8 waves, one per CU)
-  int tiles_m, tiles_n, splits, kps;
+  int shape, tiles_m, tiles_n, splits, kps;
   size_t bytes;   // workspace (0: no K slices)
 };
-using TgBig = TgShape<8, 4, 8>;
-using TgSmall = TgShape<4, 4, 4>;
-using TgTall = TgShape<4, 4, 8, 4>;   // 256 X rows x 128 W rows: waves in a 4 x 2 grid of 64 x 64 blocks
-using TgSmall8 = TgShape<4, 2, 8, 2>; // 128 x 128 with 8 waves in a 2 x 4 grid of 64 x 32 blocks
-using TgN96 = TgShape<2, 3, 8, 4>;    // 128 x 96 with 8 waves in a 4 x 2 grid of 32 x 48 blocks
-static_assert(TgSmall8::BM == TgSmall::BM && TgSmall8::BN == TgSmall::BN, "same tile, twice the waves");
-static int tg_bm(int shape) { return shape == TG_BIG ? TgBig::BM : shape == TG_TALL ? TgTall::BM : TgSmall::BM; }
-static int tg_bn(int shape) {
-  return shape == TG_BIG ? TgBig::BN : shape == TG_TALL ? TgTall::BN : shape == TG_N96 ? TgN96::BN : TgSmall::BN;
-}
-static void tg_tiles(TgPlan& p, int M, int N, bool silu) {
-  const int bm = tg_bm(p.shape), bn = tg_bn(p.shape);
-  p.tiles_m = (M + bm - 1) / bm;
-  p.tiles_n = silu ? (N / 2 + bn / 2 - 1) / (bn / 2) : (N + bn - 1) / bn;
-}
-// 256 x 256 tiles (one workgroup per CU) when there is one for every CU; otherwise 128 x 128 tiles (two per
-// CU), unsliced: K = 1536 shapes were never faster sliced. Long K (at least 128 steps, a STORE epilogue) with
-// fewer tiles than CUs: one round of at most one workgroup per CU -- a CU that runs two workgroups of a
-// launch finishes last, at about twice the time of the others -- either 128 x 128 tiles in at most
-// TG_PLAN_SPLITS K slices or 256 x 128 tiles in at most 4 (the last slice's merge reads every partial tile),
-// whichever fills more CUs, the 256 x 128 tiles on a tie (they move 25 % fewer bytes per flop through the
-// CU's load path). Each slice holds at least eight 32-wide steps. Measured, 1536 x 8960 weights (us):
-//   rows                    256   512   768  1024  1280  1552  2048
-//   128^2, slices to fill   36.0  40.6  50.0  65.2  68.8  83.5 109.6   (6, 5, 3, 2, 2, 1 (3 at 1552), 1)
-//   256 x 128, to fill        -     -     -   63.7  69.9  76.7  96.0   (4, 4, 3, 2 slices)
-//   the earlier plan (128^2 slices for two per CU)  36.0  60.6  57.6  63.9  73.0  83.0 116.8
-static inline void tg_plan_override(TgPlan&, int, int, bool, int&) {}
-static int tg_fill_splits(int tiles, int max_splits, int steps) {
-  int s = target_workgroups() / tiles;
-  if (s > max_splits) s = max_splits;
-  if (s > steps / 8) s = steps / 8;
-  return s < 1 ? 1 : s;
-}
-static TgPlan tg_plan(int M, int N, int K, int epi) {
+// The tile and K slices with the least modelled time. Slices (at least eight slabs each, one round only) pay for the
+// published partials, which the tile's last slice to finish reads back: 3 us and, per KB of partial, 38 ns for the second
+// slice and 37 for each further one (800 x 1536 x 1536: 256 x 128 tiles 24.8, 22.1, 22.0, 24.6 us in 1 .. 4 slices, 128 x
+// 128 16.1, 15.8, 17.1; 1553 x 1536 x 8960: 256 x 128 tiles 104, 65, 57 us in 1, 2, 3 slices, 128 x 128 unsliced 65, 128 x
+// 96 60; 512 rows of it: 128 x 96 tiles 57, 34, 28, 26 us in 1 .. 4 slices, 128 x 128 in 5 27). Plain,
+// residual and RoPE products of one shape take the same slices, so their sums agree bit for bit; SiLU products are not
+// sliced. A function of the shape alone, so a given call always sums in the same order.
+static inline void tg_plan_override(TgPlan&, int, int, int) {}
+static TgPlan tg_plan_of(int M, int N, int K, int epi, int sp_min, int sp_max) {
   const bool silu = epi == EPI_SILU;
-  TgPlan p;
-  const int T = target_workgroups(), steps = K / TG_BK;
-  p.shape = TG_BIG;
-  tg_tiles(p, M, N, silu);
-  if (int64_t(p.tiles_m) * p.tiles_n < T) {
-    p.shape = TG_SMALL;
-    tg_tiles(p, M, N, silu);
-  }
-  int tiles = p.tiles_m * p.tiles_n;
-  int splits = 1;
-  if (steps >= 128 && !silu && p.shape == TG_SMALL && tiles < T) {
-    const int s_small = tg_fill_splits(tiles, TG_PLAN_SPLITS, steps);
-    TgPlan t = p;
-    t.shape = TG_TALL;
-    tg_tiles(t, M, N, silu);
-    const int tt = t.tiles_m * t.tiles_n, s_tall = tt < T ? tg_fill_splits(tt, 4, steps) : 1;
-    if (tt < T && tt * s_tall >= tiles * s_small) {
-      p = t;
-      splits = s_tall;
-    } else {
-      splits = s_small;
+  const int T = target_workgroups(), slabs = (K + TG_BK - 1) / TG_BK;
+  TgPlan p{};
+  int64_t best = INT64_MAX;
+  for (int sh = 0; sh < TG_TILES; ++sh) {
+    const TgTile& t = TG_TILE[sh];
+    if ((silu && !t.silu) || (epi == EPI_ROPE && !t.rope)) continue;
+    const int tm = (M + t.bm - 1) / t.bm;
+    const int tn = silu ? (N / 2 + t.bn / 2 - 1) / (t.bn / 2) : (N + t.bn - 1) / t.bn;
+    const int64_t tiles = int64_t(tm) * tn;
+    for (int sp = sp_min; sp <= (t.split ? sp_max : 1); ++sp) {
+      if (sp > 1 && (tiles * sp > T || slabs < 8 * sp)) break;
+      const int kps = (slabs + sp - 1) / sp;
+      const int64_t rounds = (tiles * sp + T - 1) / T;
+      const int64_t cost = rounds * (int64_t(kps) * t.slab + t.fixed) + (sp > 1 ? 3000 + int64_t(t.bm) * t.bn / 256 * (38 + 37 * (sp - 2)) : 0);
+      if (cost < best) {
+        best = cost;
+        p = TgPlan{sh, tm, tn, sp, kps, 0};
+      }
     }
   }
-  // a 128 x 128 STORE plan that fits one workgroup per CU runs the 8-wave tile: two waves per SIMD instead of
-  // one, so one wave's LDS reads and barrier overlap the other's products (1552 x 1536 x 1536: 18.8 -> 17.4 us;
-  // 512 x 1536 x 8960 in 5 slices: 40.4 -> 38.0)
-  if (!silu && p.shape == TG_SMALL && tiles * splits <= T) p.shape = TG_SMALL8;
-  // ... and an unsliced one (no RoPE: its heads are 64 or 128 wide) that leaves CUs idle takes 128 x 96 tiles
-  // (8 waves of 32 x 48) when they too fit one round and cover N exactly: more CUs, each SIMD with three
-  // quarters of the work (1552 x 1536 x 1536: 19.1 -> 18.7 us, 20.0 -> 19.3 with the residual add; 300 rows
-  // 18.8 -> 17.2; 1552 x 1003 x 896, a partial last column tile: 14.3 -> 14.6, hence N % 96 == 0)
-  if ((epi == EPI_STORE || epi == EPI_RESNORM) && p.shape == TG_SMALL8 && splits == 1 && N % TgN96::BN == 0) {
-    TgPlan t = p;
-    t.shape = TG_N96;
-    tg_tiles(t, M, N, false);
-    if (t.tiles_m * t.tiles_n <= T) p = t;
-  }
-  tg_plan_override(p, M, N, silu, splits);
-  tiles = p.tiles_m * p.tiles_n;
-  if (splits > TG_MAX_SPLITS) splits = TG_MAX_SPLITS;
-  if (splits > steps) splits = steps;
-  if (splits < 1) splits = 1;
-  p.kps = (steps + splits - 1) / splits;
-  p.splits = (steps + p.kps - 1) / p.kps;   // every slice non-empty
-  const int part = tg_bm(p.shape) * tg_bn(p.shape);
-  p.bytes = p.splits > 1 ? G_CNT_BYTES + align256(sizeof(float) * size_t(tiles) * p.splits * part) : 0;
+  return p;
+}
+static TgPlan tg_plan(int M, int N, int K, int epi) {
+  TgPlan p = tg_plan_of(M, N, K, epi == EPI_SILU ? epi : EPI_STORE, 1, epi == EPI_SILU ? 1 : TG_MAX_SPLITS);
+  // (128 x 96 tiles, the only ones that RoPE's heads do not fit, are the smallest: any other tile keeps within the round)
+  if (epi == EPI_ROPE) p = tg_plan_of(M, N, K, epi, p.splits, p.splits);
+  const int slabs = (K + TG_BK - 1) / TG_BK;
+  tg_plan_override(p, M, N, epi);
+  p.splits = (slabs + p.kps - 1) / p.kps;   // every slice non-empty
+  if (p.splits > 1)
+    p.bytes = G_CNT_BYTES + align256(sizeof(float) * size_t(p.tiles_m) * p.tiles_n * p.splits * TG_TILE[p.shape].bm * TG_TILE[p.shape].bn);
   return p;
 }
 static TgArgs tg_args(const void* x, const void* w, const void* bias, void* y, int M, int N, int K) {
@@ -1832,7 +1896,6 @@ static int launch_tiled(TgArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
   NS_REQUIRE((int64_t(M) + 256) * K * 2 < (int64_t(1) << 31) && (int64_t(N) + 256) * K * 2 < (int64_t(1) << 31),
              "gemm: X [%d, %d] or W [%d, %d] too large for 32-bit buffer offsets", M, K, N, K);
   const TgPlan p = tg_plan(M, N, K, EPI);
-  NS_REQUIRE(EPI != EPI_ROPE || (tg_bn(p.shape) % a.hd == 0), "gemm(tiled): head_dim %d does not divide the tile", a.hd);
   a.tiles_m = p.tiles_m;
   a.tiles_n = p.tiles_n;
   a.splits = p.splits;
@@ -1848,19 +1911,16 @@ static int launch_tiled(TgArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
     a.part = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + G_CNT_BYTES);
   }
   const dim3 grid(unsigned(p.tiles_m * p.tiles_n * p.splits));
-  constexpr int EPIT = EPI == EPI_SILU ? EPI_STORE : EPI;   // the 256 x 128 and 8-wave 128^2 tiles: no SiLU
-  if (p.shape == TG_BIG)
-    hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 8, 4, 8, 2>), grid, dim3(TgBig::NT), 0, st, a);
-  else if (EPI != EPI_SILU && p.shape == TG_TALL)
-    hipLaunchKernelGGL((tiled_gemm_kernel<EPIT, 4, 4, 8, 4>), grid, dim3(TgTall::NT), 0, st, a);
-  else if (EPI != EPI_SILU && p.shape == TG_SMALL8)
-    hipLaunchKernelGGL((tiled_gemm_kernel<EPIT, 4, 2, 8, 2>), grid, dim3(TgSmall8::NT), 0, st, a);
-  else if (p.shape == TG_N96) {
-    if constexpr (EPI == EPI_STORE || EPI == EPI_RESNORM)
-      hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 2, 3, 8, 4>), grid, dim3(TgN96::NT), 0, st, a);
+  const dim3 threads(512);
+  constexpr int EPI_TALL = EPI == EPI_SILU ? EPI_STORE : EPI, EPI_96 = EPI == EPI_RESNORM ? EPI : EPI_STORE;
+  switch (p.shape) {   // the plan keeps SILU off the 256 x 128 and 128 x 96 tiles, and ROPE off the latter
+    case TG_256x256: hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 8, 4, 2>), grid, threads, 0, st, a); break;
+    case TG_192x256: hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 6, 4, 2>), grid, threads, 0, st, a); break;
+    case TG_128x256: hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 4, 4, 2>), grid, threads, 0, st, a); break;
+    case TG_256x128: hipLaunchKernelGGL((tiled_gemm_kernel<EPI_TALL, 4, 4, 4>), grid, threads, 0, st, a); break;
+    case TG_128x128: hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 2, 4, 4>), grid, threads, 0, st, a); break;
+    default: hipLaunchKernelGGL((tiled_gemm_kernel<EPI_96, 2, 3, 4>), grid, threads, 0, st, a); break;
   }
-  else
-    hipLaunchKernelGGL((tiled_gemm_kernel<EPI, 4, 4, 4, 2>), grid, dim3(TgSmall::NT), 0, st, a);
   return check_launch("gemm(tiled)");
 }
 
@@ -1894,13 +1954,13 @@ static size_t skinny_large_m_bytes(const Plan& p, int mblocks) {
 extern "C" size_t ns_gemm_workspace_bytes(int M, int N, int K) {
   if (M < 1 || N < 1 || K < 32) return 0;
   if (M > G_MAX_M) {
-    size_t a = tg_plan(M, N, K, EPI_STORE).bytes, b = tg_plan(M, N, K, EPI_SILU).bytes;
+    size_t a = tg_plan(M, N, K, EPI_STORE).bytes;   // only plain and residual products are sliced, and alike
     // the 64-row token blocks of the skinny kernel (STORE with long K; residual + statistics at any K)
     if (M <= t16_max_m() && (M + G_MAX_M - 1) / G_MAX_M * ((N + 63) / 64) <= G_MAX_TILES) {
       const size_t c = skinny_large_m_bytes(make_plan((N + 63) / 64, K), (M + G_MAX_M - 1) / G_MAX_M);
       a = a > c ? a : c;
     }
-    return a > b ? a : b;
+    return a;
   }
   return make_plan((N + 63) / 64, K).bytes;
 }

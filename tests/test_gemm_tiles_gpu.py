@@ -1,0 +1,75 @@
+"""The tiled GEMM's tile shapes at their edges: row and column remainders, a last slab of 32 k, K slices of unequal
+length, every epilogue. Plain products against the fp32-accumulated, once-rounded product (a bf16 ulp plus the
+dot-product bound of both sides); the fused epilogues bitwise against the plain product followed by the unfused op."""
+import pytest
+import torch
+
+from oracle import ops
+from tests.conftest import cpu_gen
+from tests.test_gemm_kernels import BF, bf16_check, dot_bound, operands, ref_linear
+
+pytestmark = pytest.mark.gpu
+
+# rows, weight rows, K: by the plan's costs on 256 x 256, 192 x 256, 128 x 256, 256 x 128, 128 x 128 and 128 x 96 tiles,
+# each with partial last tiles, and 128 x 96 and 256 x 128 tiles in several K slices
+SHAPES = [(1530, 10248, 96), (2300, 5000, 160), (380, 21000, 96), (4000, 1032, 4096), (1280, 3208, 224), (700, 1528, 416),
+          (300, 1032, 2080), (1553, 1536, 8992), (65, 20000, 96)]
+
+
+def edge_rows(M):
+    return torch.tensor(sorted({r for t in (96, 128, 192, 256) for t0 in range(0, M, t) for r in (t0, t0 + t // 2 - 1, t0 + t - 1)
+                                if r < M} | {M - 1})[::3] + [M - 1])
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_store_and_residual(hiplib, M, N, K):
+    from nanoserve_amd.kernels.linear import linear, linear_residual_rms_norm
+    x, w = operands(M, N, K, seed=M + N)
+    b = (torch.randn(N, generator=cpu_gen(1)) * 0.1).to(BF)
+    dx, dw = x.cuda(), w.cuda()
+    y = linear(dx, dw, b.cuda())
+    rows = edge_rows(M)
+    bf16_check(y.cpu()[rows], ref_linear(x[rows], w, b), f"tiled linear {M} x {N} x {K}", dot_bound(x[rows], w))
+    assert torch.equal(y, linear(dx, dw, b.cuda()))
+    if M > 192:   # the residual epilogue's range
+        res = torch.randn(M, N, generator=cpu_gen(2)).to(BF).cuda()
+        total = linear_residual_rms_norm(dx, dw, res, None, 1e-6)[1]
+        assert torch.equal(total, res + linear(dx, dw))
+
+
+@pytest.mark.parametrize("M,half,K", [(1530, 5124, 96), (2300, 2500, 160), (257, 8188, 96), (700, 768, 416), (65, 10000, 96),
+                                      (129, 100, 32), (193, 1001, 64)])
+def test_silu(hiplib, M, half, K):
+    from nanoserve_amd.kernels.linear import linear_silu_mul
+    x, w = operands(M, 2 * half, K, seed=M + half)
+    out = linear_silu_mul(x.cuda(), w.cuda()).cpu()
+    rows = edge_rows(M)
+    acc = x[rows].double() @ w.double().t()
+    g, u = acc[:, :half].float(), acc[:, half:].float()
+    ref = ops.silu_mul(torch.cat([g.to(BF), u.to(BF)], dim=1)).float()
+    # a gate or up value may round the other way (2^-8 of it), the SiLU and the product round once more each
+    scale = (g.abs() + 1) * (u.abs() + 1)
+    assert ((out[rows].float() - ref).abs() <= 2.0 ** -6 * scale).all()
+    assert (out[rows].float() - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K", [(1530, 78, 2, 128, 96), (4090, 14, 2, 64, 96), (2300, 28, 6, 128, 96), (380, 160, 2, 128, 96),
+                                           (300, 16, 2, 128, 2080), (700, 5, 1, 64, 224), (6000, 12, 2, 128, 160)])
+def test_rope(hiplib, M, nh, nkv, hd, K):
+    from nanoserve_amd.kernels.fused import rope_qkv
+    from nanoserve_amd.kernels.linear import linear, linear_rope_qkv
+    N = (nh + 2 * nkv) * hd
+    x, w = operands(M, N, K, seed=M + hd)
+    g = cpu_gen(M)
+    b = (torch.randn(N, generator=g) * 0.1).to(BF).cuda()
+    cos, sin = (t.cuda() for t in ops.rope_tables(torch.randint(0, 32768, (M,), generator=g), hd, 1e6, BF))
+    slots = torch.randperm((M // 16 + 2) * 16, generator=g)[:M].cuda()
+    for bias, cached in ((b, True), (None, False)):
+        caches = [[torch.zeros(M // 16 + 2, 16, nkv, hd, dtype=BF, device="cuda") for _ in range(2)] if cached else [None, None]
+                  for _ in range(2)]
+        fused = linear_rope_qkv(x.cuda(), w.cuda(), bias, cos, sin, nh, nkv, hd, *caches[0], slots if cached else None)
+        plain = rope_qkv(linear(x.cuda(), w.cuda(), bias), cos, sin, nh, nkv, hd, *caches[1], slots if cached else None)
+        for a, r in zip(fused, plain):
+            assert torch.equal(a, r)
+        if cached:
+            assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
