@@ -863,7 +863,7 @@ __global__ __launch_bounds__(ROWK_NW * 64) void paged_decode_rows_bf16_kernel(Ro
 // prefill units that found no free CU started ~10 us late and the launch took 37 us against 28 us for the
 // prefill alone. Two streams overlap them too, but a graph's cross-queue fork and join idle the GPU for
 // longer than that saves.)
-template <int HD, bool PH>
+template <int HD, bool PH, bool MANY>
 __global__ __launch_bounds__(PF_WG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void mixed_attn_kernel(
     PrefillArgs pa, int n_pf, RowsArgs ra) {
   static_assert(PF_WG_THREADS == ROWK_NW * 64, "one workgroup size for both kinds");
@@ -873,7 +873,7 @@ __global__ __launch_bounds__(PF_WG_THREADS) __attribute__((amdgpu_waves_per_eu(2
   __shared__ float sm_m[ROWK_NW][16], sm_l[ROWK_NW][16];
   __shared__ unsigned s_last;
   if (int(blockIdx.x) < n_pf)
-    prefill_body<HD>(pa, int(blockIdx.x), lds, s_last);
+    prefill_workgroup<HD, MANY>(pa, int(blockIdx.x), lds, s_last);
   else
     decode_rows_body<HD, PH>(ra, int(blockIdx.x) - n_pf, lds, sm_m, sm_l, s_last);
 }
@@ -1281,6 +1281,15 @@ extern "C" int ns_paged_attn_decode_rows(const void* q, int64_t q_sb, int64_t q_
                              num_blocks, scale, dtype, workspace, workspace_bytes, stream, q_rows);
 }
 
+static void launch_mixed(int head_dim, bool per_head, dim3 grid, hipStream_t s, const PrefillArgs& pa, int n_pf, const RowsArgs& ra) {
+  const bool many = prefill_many(pa);
+  const auto kernel =
+      head_dim == 64 ? (many ? mixed_attn_kernel<64, false, true> : mixed_attn_kernel<64, false, false>)
+      : per_head     ? (many ? mixed_attn_kernel<128, true, true> : mixed_attn_kernel<128, true, false>)
+                     : (many ? mixed_attn_kernel<128, false, true> : mixed_attn_kernel<128, false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(PF_WG_THREADS), 0, s, pa, n_pf, ra);
+}
+
 extern "C" int ns_paged_attn_mixed(const void* q, int64_t q_sb, int64_t q_sh, const void* k_pool, const void* v_pool,
                                    int64_t kv_sblk, int64_t kv_spos, int64_t kv_sh, const int32_t* pf_block_tables,
                                    int64_t pf_bt_sb, const int32_t* seq_info, int n_seqs, int max_new, int max_kv,
@@ -1310,11 +1319,7 @@ extern "C" int ns_paged_attn_mixed(const void* q, int64_t q_sb, int64_t q_sh, co
   if (n_pf == 0 || rl.grid == 0) {   // one side only: its own kernel
     if (rl.grid > 0) launch_rows(rl.a, rl.grid, rl.rgh, rl.head_dim, s);
     if (n_pf > 0) {
-      const dim3 grid{unsigned(n_pf)};
-      if (head_dim == 64)   // every workgroup a prefill one
-        hipLaunchKernelGGL((mixed_attn_kernel<64, false>), grid, dim3(PF_WG_THREADS), 0, s, pa, int(n_pf), rl.a);
-      else
-        hipLaunchKernelGGL((mixed_attn_kernel<128, false>), grid, dim3(PF_WG_THREADS), 0, s, pa, int(n_pf), rl.a);
+      launch_mixed(head_dim, false, dim3{unsigned(n_pf)}, s, pa, int(n_pf), rl.a);   // every workgroup a prefill one
     }
     return check_launch("paged_attention_mixed");
   }
@@ -1325,12 +1330,7 @@ extern "C" int ns_paged_attn_mixed(const void* q, int64_t q_sb, int64_t q_sh, co
              (long long)(n_pf8 + rl.grid));
   const dim3 grid{unsigned(n_pf8 + rl.grid)};
   const int npf = int(n_pf8);
-  if (rl.rgh > 1)
-    hipLaunchKernelGGL((mixed_attn_kernel<128, true>), grid, dim3(PF_WG_THREADS), 0, s, pa, npf, rl.a);
-  else if (rl.head_dim == 64)
-    hipLaunchKernelGGL((mixed_attn_kernel<64, false>), grid, dim3(PF_WG_THREADS), 0, s, pa, npf, rl.a);
-  else
-    hipLaunchKernelGGL((mixed_attn_kernel<128, false>), grid, dim3(PF_WG_THREADS), 0, s, pa, npf, rl.a);
+  launch_mixed(rl.head_dim, rl.rgh > 1, grid, s, pa, npf, rl.a);
   return check_launch("paged_attention_mixed");
 }
 

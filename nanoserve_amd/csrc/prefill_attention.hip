@@ -4,11 +4,11 @@
 namespace ns {
 namespace {
 
-template <int HD>
+template <int HD, bool MANY>
 __global__ __launch_bounds__(PF_WG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void paged_prefill_bf16_kernel(PrefillArgs a) {
   __shared__ __align__(16) unsigned char lds[PF_GROUPS * 2 * PfLds<HD>::STAGE];
   __shared__ unsigned s_last;
-  prefill_body<HD>(a, int(blockIdx.x), lds, s_last);
+  prefill_workgroup<HD, MANY>(a, int(blockIdx.x), lds, s_last);
 }
 
 }  // namespace
@@ -37,9 +37,9 @@ extern "C" int ns_paged_attn_prefill(const void* q, int64_t q_st, int64_t q_sh, 
   if (st != NS_OK || n_wg == 0) return st;
   const dim3 grid{unsigned(n_wg)};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (head_dim == 64)
-    hipLaunchKernelGGL(paged_prefill_bf16_kernel<64>, grid, dim3(PF_WG_THREADS), 0, s, a);
-  else
-    hipLaunchKernelGGL(paged_prefill_bf16_kernel<128>, grid, dim3(PF_WG_THREADS), 0, s, a);
+  const bool many = prefill_many(a);
+  const auto kernel = head_dim == 64 ? (many ? paged_prefill_bf16_kernel<64, true> : paged_prefill_bf16_kernel<64, false>)
+                                     : (many ? paged_prefill_bf16_kernel<128, true> : paged_prefill_bf16_kernel<128, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(PF_WG_THREADS), 0, s, a);
   return check_launch("paged_attention_prefill");
 }

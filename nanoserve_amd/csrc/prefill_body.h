@@ -164,10 +164,24 @@ struct PrefillArgs {
   float* ws_acc;                    // [unit][R][NT][256 threads] float4
 };
 
-// The kernel's body: bid is the workgroup's index among the prefill workgroups of the launch; lds the
+// How a workgroup reads seq_info: from memory, or a sequence per lane (PF_LANE_SEQS at most, one load for all of them).
+struct PfInfoMem {
+  __device__ __forceinline__ int q_start(const PrefillArgs& a, int s) const { return a.info[4 * s + 0]; }
+  __device__ __forceinline__ int n_new(const PrefillArgs& a, int s) const { return a.info[4 * s + 1]; }
+  __device__ __forceinline__ int ctx(const PrefillArgs& a, int s) const { return a.info[4 * s + 2]; }
+};
+constexpr int PF_LANE_SEQS = 64;
+struct PfInfoLanes {
+  int row, new_, ctx_;
+  __device__ __forceinline__ int q_start(const PrefillArgs&, int s) const { return __builtin_amdgcn_readlane(row, s); }
+  __device__ __forceinline__ int n_new(const PrefillArgs&, int s) const { return __builtin_amdgcn_readlane(new_, s); }
+  __device__ __forceinline__ int ctx(const PrefillArgs&, int s) const { return __builtin_amdgcn_readlane(ctx_, s); }
+};
+
+// The kernel's body for few tiles: bid is the workgroup's index among the prefill workgroups of the launch; lds the
 // launch's LDS (at least PF_GROUPS * 2 * PfLds<HD>::STAGE bytes, 16-byte aligned) and s_last one LDS word.
-template <int HD>
-__device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsigned char* lds, unsigned& s_last) {
+template <int HD, class Info>
+__device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Info& seqs, int bid, unsigned char* lds, unsigned& s_last) {
   using L = PfLds<HD>;
   constexpr int KS = HD / 32;   // k-steps of Q.K^T
   constexpr int NT = HD / 16;   // output tiles of P.V
@@ -181,7 +195,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsi
   // (group 1). A sequence with more new tokens than the caller's max_new is not computed.
   int rem = bid, seq = -1, tile = 0, part = 0, h = 0, n_st = 0, n_parts = 0, n_pages = 0;
   for (int sq = 0; sq < a.n_seqs && seq < 0; ++sq) {
-    const int Tq = a.info[4 * sq + 1], cq = a.info[4 * sq + 2];
+    const int Tq = seqs.n_new(a, sq), cq = seqs.ctx(a, sq);
     const int nt = (Tq + PF_QT - 1) / PF_QT;
     if (Tq <= 0 || nt > a.tiles_max) continue;
     for (int tr = 0; tr < nt; ++tr) {
@@ -203,7 +217,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsi
     }
   }
   if (seq < 0) return;
-  const int q_start = a.info[4 * seq + 0], T = a.info[4 * seq + 1], ctx = a.info[4 * seq + 2];
+  const int q_start = seqs.q_start(a, seq), T = seqs.n_new(a, seq), ctx = seqs.ctx(a, seq);
   const int qbase = tile * PF_QT;
   const int kv_total = ctx + T;             // keys that exist
   const int n_sub = 2 * n_parts;
@@ -283,6 +297,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsi
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[rt][t] = pf_float4_t{0.f, 0.f, 0.f, 0.f};
   }
+
+  const int v_row = 4 * r4 + (c16 >> 2);   // the key row (of a page) this lane addresses in V reads
+  const uint32_t v_off = uint32_t(v_row * L::ROW + 16 * (((c16 & 3) >> 1) ^ L::vkey(v_row)) + 8 * (c16 & 1));
 
   // One stage: S^T for all 64 keys (both halves of 32 keys: pages 2 hs, 2 hs + 1), one softmax update
   // per query tile over the whole stage, then P and O^T += V^T . P^T half by half, with the second half's
@@ -371,8 +388,6 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsi
 #pragma unroll
       for (int hp = 0; hp < 2; ++hp) {
         const int pp = 2 * hs + hp;
-        const int vr = PF_PAGE * pp + 4 * r4 + (c16 >> 2);   // the key row this lane addresses
-        const unsigned char* vrow = st + L::K_BYTES + vr * L::ROW;
         uint32_t m01 = 0xffffffffu, m23 = 0xffffffffu;
         if constexpr (MODE == 2) {
           const int key0 = kb0 + PF_PAGE * pp + 4 * r4;
@@ -382,9 +397,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsi
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          const int dim = 16 * t + 4 * (c16 & 3);
-          const int chunk = dim >> 3;
-          const unsigned char* src = vrow + 16 * (chunk ^ L::vkey(vr)) + 2 * (dim & 7);
+          const unsigned char* src = st + L::K_BYTES + PF_PAGE * L::ROW * pp + (v_off ^ uint32_t(32 * t));
           v4i16_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4i16_t*)(src));
           if constexpr (MODE == 2) {
             uint2 u = __builtin_bit_cast(uint2, v);
@@ -676,6 +689,428 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, int bid, unsi
   if (gi == 0) merge_half(G0{}); else merge_half(G1{});
   __syncthreads();
   store_tile();
+}
+
+// ---------------------------------------------------------------------------------------------------
+// Many query tiles in the launch (prefill_workgroup decides): a workgroup takes two tiles that read the same K and V -- two neighbouring
+// heads of a KV head, or, with an odd number of them, two neighbouring query tiles of a head -- over all their keys,
+// instead of one tile's keys in two ranges. Then
+//   * both groups share the stages: half the copies, four slots of K and V, copies issued two and three stages ahead;
+//   * nothing is merged at the end;
+//   * the groups run in opposite phases. Per 64-key stage n a wave has a vector half (reads the K fragments of stage
+//     n + 1, issues its copies, softmax of the scores of stage n) and a matrix half (scores of stage n + 1, P.V of stage
+//     n), a barrier after each; group 1 starts half a stage late, so of the two waves of a SIMD (w and w + 4) one
+//     multiplies while the other is in its exponentials.
+// Slot safety: K (n + 3) replaces K (n - 1), read by both groups before the barrier that starts group 0's vector half n,
+// and V (n + 2) replaces V (n - 2), likewise. Each wave waits for its copies of K (n + 1) and V (n) before the barrier that
+// precedes group 0's vector half n: group 0 at the end of its matrix half n - 1, group 1 at the end of its vector half
+// n - 1. The sums of a tile run over its stages in order; the arithmetic of a stage is prefill_body's.
+// Bound: per stage and CU 2048 cycles of products per SIMD, about 1400 of vector work and 2300 of LDS traffic.
+constexpr int PF_SLOTS_KV = 4;     // LDS slots of K and of V
+constexpr int PF_CUS = 256;
+
+template <int HD>
+__device__ __forceinline__ void prefill_pair_body(const PrefillArgs& a, const PfInfoLanes& seqs, int bid, unsigned char* lds) {
+  using L = PfLds<HD>;
+  constexpr int KS = HD / 32, NT = HD / 16;
+  constexpr int KB = L::K_BYTES;   // bytes of a K or V slot
+  const int tid_wg = threadIdx.x, lane = tid_wg & 63, w8 = __builtin_amdgcn_readfirstlane(tid_wg >> 6);
+  const int gi = w8 >> 2, w = w8 & 3;
+  const int c16 = lane & 15, r4 = lane >> 4;
+
+  // ---- the unit. Tiles (of qt queries: 128 by head pairs, 256 by tile pairs) go from those with the most keys to those
+  // with the fewest over all sequences, so the launch ends on short ones. Lane s counts, in closed form, sequence s's
+  // tiles whose last key lies in 64-key stage x or later; the sum over the lanes is searched for the stage that holds
+  // this unit, then the lanes for its sequence. (A stage holds at most two tiles of a sequence.)
+  const bool by_head = (a.G & 1) == 0;   // pairs of heads; else pairs of query tiles
+  const int qt = by_head ? PF_QT : 2 * PF_QT, per = by_head ? a.n_heads / 2 : a.n_heads;
+  const int my_T = lane < a.n_seqs && seqs.new_ > 0 && (seqs.new_ + PF_QT - 1) / PF_QT <= a.tiles_max ? seqs.new_ : 0;
+  const int my_ctx = seqs.ctx_, my_nt = (my_T + qt - 1) / qt;
+  auto tiles_from = [&](int x) __attribute__((always_inline)) {   // this lane's tiles with keys in stage x or later
+    if (my_T == 0) return 0;
+    const int first = max((PF_KEYS * x + 1 - my_ctx + qt - 1) >> (by_head ? 7 : 8), 1);   // whole tiles first .. my_nt - 1
+    return min(max(my_nt - first, 0), my_nt - 1) + ((my_ctx + my_T - 1) / PF_KEYS >= x ? 1 : 0);
+  };
+  auto sum_lanes = [&](int v) __attribute__((always_inline)) {
+    int sum = 0;
+    for (int s = 0; s < a.n_seqs; ++s) sum += __builtin_amdgcn_readlane(v, s);
+    return sum;
+  };
+  int x = 0, x_end = 0;   // the stage: units from x on > bid >= units from x + 1 on
+  for (int s = 0; s < a.n_seqs; ++s) {
+    const int last = __builtin_amdgcn_readlane(my_T > 0 ? my_ctx + my_T : 0, s);
+    x_end = max(x_end, (last + PF_KEYS - 1) / PF_KEYS);
+  }
+  if (bid >= sum_lanes(tiles_from(0)) * per) return;
+  while (x_end - x > 1) {
+    const int mid = (x + x_end) >> 1;
+    if (sum_lanes(tiles_from(mid)) * per > bid) x = mid; else x_end = mid;
+  }
+  const int my_later = tiles_from(x + 1), my_here = tiles_from(x) - my_later;
+  int rem = bid - sum_lanes(my_later) * per, seq = 0, nth = 0;
+  for (int s = 0; s < a.n_seqs; ++s) {
+    const int units = __builtin_amdgcn_readlane(my_here, s) * per;
+    if (rem < units) {
+      seq = s;
+      nth = rem / per;
+      break;
+    }
+    rem -= units;
+  }
+  const int hx = rem - nth * per;
+  // counted from the sequence's last tile: its tiles in later stages, then nth of this stage
+  const int lev = __builtin_amdgcn_readlane(my_nt, seq) - 1 - __builtin_amdgcn_readlane(my_later, seq) - nth;
+  const int tile = by_head ? lev : 2 * lev + gi, tile_hi = by_head ? lev : 2 * lev + 1;   // tile_hi: the later of the two
+  const int h = by_head ? 2 * hx + gi : hx;
+  const int g = h / a.G;
+  const int q_start = seqs.q_start(a, seq), T = seqs.n_new(a, seq), ctx = seqs.ctx(a, seq);
+  const int kv_total = ctx + T;
+  const int n_pages = min((ctx + min(PF_QT * (tile_hi + 1), T) + PF_PAGE - 1) / PF_PAGE, a.max_blocks);
+  const int n_st = (n_pages + PF_NP - 1) / PF_NP;
+  const int32_t* table = a.bt + int64_t(seq) * a.bt_sb;
+  const int qbase = tile * PF_QT;
+
+  pf_bf16x8_t qf[PF_R][KS];
+  auto jrow = [&](int rt) __attribute__((always_inline)) {   // rows past T mirror row T - 1 and are not stored
+    return min(qbase + 16 * PF_R * w + 16 * rt + c16, T - 1);
+  };
+#pragma unroll
+  for (int rt = 0; rt < PF_R; ++rt) {
+    const bf16_t* qrow = a.q + int64_t(q_start + jrow(rt)) * a.q_st + int64_t(h) * a.q_sh;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      qf[rt][s] = __builtin_bit_cast(pf_bf16x8_t, *reinterpret_cast<const uint4*>(qrow + 32 * s + 8 * r4));
+  }
+  const int j_first_w = qbase + 16 * PF_R * w, j_last_w = min(j_first_w + 16 * PF_R - 1, T - 1);
+  // stages in which the wave sees a key (its queries' last visible key ends them)
+  const int n_act = j_first_w < T ? min(n_st, (ctx + j_last_w) / PF_KEYS + 1) : 0;
+
+  // ---- copies: a window of 64 table entries, one per lane; wave w8 copies half w8 & 1 of page w8 >> 1 of a stage
+  int win0 = 0, pid = 0;
+  uint64_t pok = 0;
+  auto load_window = [&](int n0) __attribute__((always_inline)) {
+    win0 = n0;
+    const int p = PF_NP * n0 + lane;
+    const int id = table[min(p, n_pages - 1)];
+    pok = __ballot(p < n_pages && id >= 0 && id < a.num_blocks);
+    pid = (id >= 0 && id < a.num_blocks) ? id : 0;   // masked pages read block 0 (in bounds)
+  };
+  auto stage_ok = [&](int n) __attribute__((always_inline)) { return unsigned(pok >> (PF_NP * (n - win0))) & 0xFu; };
+  const uint32_t lds0 = pf_lds_addr(lds);
+  const uint32_t spos2 = uint32_t(a.s_pos) * 2u;
+  constexpr int HI = L::IPP / 2;   // loads per wave, stage and tensor
+  const int i0 = HI * (w8 & 1);
+  // the wave's loads start at token row TPI i0 of the page, whose swizzle keys they share (keys split over the sum)
+  const uint32_t lane_row = uint32_t(lane / L::CH) * spos2;
+  const uint32_t lane_kx = 16u * uint32_t((lane % L::CH) ^ L::key(lane / L::CH) ^ L::key(L::TPI * i0));
+  const uint32_t lane_vx = 16u * uint32_t((lane % L::CH) ^ L::vkey(lane / L::CH) ^ L::vkey(L::TPI * i0));
+  auto copy = [&](int n, bool is_v) __attribute__((always_inline)) {
+    const int id = __builtin_amdgcn_readlane(pid, PF_NP * (n - win0) + (w8 >> 1));
+    const int64_t base = (int64_t(id) * a.s_blk + int64_t(g) * a.s_h) * 2 + int64_t(L::TPI * i0) * spos2;
+    const char* src = reinterpret_cast<const char*>(is_v ? a.vp : a.kp) + base;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(
+        lds0 + uint32_t((n & (PF_SLOTS_KV - 1)) * KB + (is_v ? PF_SLOTS_KV * KB : 0) + (w8 >> 1) * (PF_PAGE * L::ROW) + 1024 * i0));
+    uint32_t lrow = lane_row, kvx = is_v ? lane_vx : lane_kx;
+    asm volatile("" : "+v"(lrow), "+v"(kvx));
+#pragma unroll
+    for (int i = 0; i < HI; ++i) {   // the keys of rows TPI (i0 + i): key(TPI i0) ^ key(TPI i) for the strides used here
+      const uint32_t x = kvx ^ uint32_t(16 * (is_v ? L::vkey(L::TPI * i) : L::key(L::TPI * i)));
+      pf_dma16(src + int64_t(L::TPI * i) * spos2, lrow + x, dst + 1024 * i);
+    }
+  };
+  static_assert(L::IPP % 2 == 0, "two waves share a page");
+
+  float m_run[PF_R], l_run[PF_R], mc[PF_R];
+  pf_float4_t acc[PF_R][NT], sc[2][PF_R][2];
+  pf_bf16x8_t kf[4][KS], pbv[2][PF_R];
+#pragma unroll
+  for (int rt = 0; rt < PF_R; ++rt) {
+    m_run[rt] = -INFINITY;
+    l_run[rt] = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[rt][t] = pf_float4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  // Fragment read offsets: the chunk index is XORed with the row's key, so a fragment's k-step or tile is an XOR on one
+  // lane offset. (Opaque copies: hoisted out of the loop, the dozen offsets would spill.)
+  const uint32_t k_off = uint32_t(c16 * L::ROW + 16 * (r4 ^ L::key(c16)));
+  const int v_row = 4 * r4 + (c16 >> 2);   // the key row (of a page) this lane addresses
+  const uint32_t v_off = uint32_t(v_row * L::ROW + 16 * (((c16 & 3) >> 1) ^ L::vkey(v_row)) + 8 * (c16 & 1));
+  auto read_k = [&](int n, int p0) __attribute__((always_inline)) {   // K fragments of pages p0, p0 + 1
+    uint32_t o = k_off;
+    asm volatile("" : "+v"(o));
+    const unsigned char* st = lds + (n & (PF_SLOTS_KV - 1)) * KB;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const unsigned char* at = st + (o ^ uint32_t(64 * s));
+#pragma unroll
+      for (int p = p0; p < p0 + 2; ++p)
+        kf[p][s] = __builtin_bit_cast(pf_bf16x8_t, *reinterpret_cast<const uint4*>(at + PF_PAGE * L::ROW * p));
+    }
+  };
+  auto scores = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = p0; p < p0 + 2; ++p)
+#pragma unroll
+      for (int rt = 0; rt < PF_R; ++rt) sc[p >> 1][rt][p & 1] = pf_float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int p = p0; p < p0 + 2; ++p)
+#pragma unroll
+        for (int rt = 0; rt < PF_R; ++rt)
+          sc[p >> 1][rt][p & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[p][s], qf[rt][s], sc[p >> 1][rt][p & 1], 0, 0, 0);
+  };
+  // scores of keys past a query's diagonal, or of pages that hold none -> -inf
+  auto mask = [&](int kb0, unsigned okm) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rt = 0; rt < PF_R; ++rt)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int lim = ((okm >> p) & 1u) != 0 ? ctx + jrow(rt) - (kb0 + PF_PAGE * p + 4 * r4) : -1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[p >> 1][rt][p & 1][e] = e <= lim ? sc[p >> 1][rt][p & 1][e] : -INFINITY;
+      }
+  };
+  auto softmax = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int rt = 0; rt < PF_R; ++rt) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, sc[p >> 1][rt][p & 1][e]);
+      mx = pf_max4(mx);
+      const float mxc = mx * a.scale_log2;
+      const bool move = mxc > m_run[rt] + PF_SLACK;
+      const float m_new = move ? mxc : m_run[rt];
+      mc[rt] = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m_run[rt] - mc[rt]);
+      m_run[rt] = m_new;
+      l_run[rt] *= alpha;
+      if (__ballot(move)) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[rt][t] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+      for (int rt = 0; rt < PF_R; ++rt) {
+        float psum = 0.f;
+        uint32_t pb[4];
+#pragma unroll
+        for (int hp = 0; hp < 2; ++hp) {
+          float pv[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[hs][rt][hp][e], a.scale_log2, -mc[rt]));
+            psum += pv[e];
+          }
+          pb[2 * hp + 0] = pf_bf16x2(pv[0], pv[1]);
+          pb[2 * hp + 1] = pf_bf16x2(pv[2], pv[3]);
+        }
+        l_run[rt] += psum;
+        // (pinned here: left alone, the compiler sinks the exponentials into the matrix half)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(pb[e]));
+        pbv[hs][rt] = __builtin_bit_cast(pf_bf16x8_t, make_uint4(pb[0], pb[1], pb[2], pb[3]));
+      }
+  };
+  // V^T fragments of pages 2 hs, 2 hs + 1 by transpose reads, and O^T += V^T . P^T over them
+  v4i16_t va[2][NT];
+  auto read_v = [&](int n, int hs) __attribute__((always_inline)) {
+    uint32_t o = v_off;
+    asm volatile("" : "+v"(o));
+    const unsigned char* st = lds + (PF_SLOTS_KV + (n & (PF_SLOTS_KV - 1))) * KB + PF_PAGE * L::ROW * 2 * hs;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const unsigned char* at = st + (o ^ uint32_t(32 * t));
+#pragma unroll
+      for (int hp = 0; hp < 2; ++hp)
+        va[hp][t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4i16_t*)(at + PF_PAGE * L::ROW * hp));
+    }
+  };
+  auto values = [&](int n, int hs, unsigned okm, bool zero) __attribute__((always_inline)) {
+    if (zero) {   // keys that do not exist read as 0
+#pragma unroll
+      for (int hp = 0; hp < 2; ++hp) {
+        const int pp = 2 * hs + hp, key0 = n * PF_KEYS + PF_PAGE * pp + 4 * r4;
+        const bool ok = ((okm >> pp) & 1u) != 0;
+        const uint32_t m01 = (ok && key0 + 0 < kv_total ? 0x0000ffffu : 0u) | (ok && key0 + 1 < kv_total ? 0xffff0000u : 0u);
+        const uint32_t m23 = (ok && key0 + 2 < kv_total ? 0x0000ffffu : 0u) | (ok && key0 + 3 < kv_total ? 0xffff0000u : 0u);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          uint2 u = __builtin_bit_cast(uint2, va[hp][t]);
+          u.x &= m01;
+          u.y &= m23;
+          va[hp][t] = __builtin_bit_cast(v4i16_t, u);
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const uint2 lo = __builtin_bit_cast(uint2, va[0][t]), hi = __builtin_bit_cast(uint2, va[1][t]);
+      const pf_bf16x8_t vav = __builtin_bit_cast(pf_bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+#pragma unroll
+      for (int rt = 0; rt < PF_R; ++rt) acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vav, pbv[hs][rt], acc[rt][t], 0, 0, 0);
+    }
+  };
+  auto barrier = [&]() __attribute__((always_inline)) {   // LDS reads done; copies may be in flight
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int AHEAD = 2 * HI;   // copies a wave issues per stage (vmcnt immediates: vmcnt(n), the rest at their maxima)
+
+  // ---- prologue: K 0 .. 2, V 0 .. 1 on their way, then the scores of stage 0
+  load_window(0);
+  unsigned ok0 = stage_ok(0), ok1 = n_st > 1 ? stage_ok(1) : 0, ok2 = n_st > 2 ? stage_ok(2) : 0;
+  copy(0, false);
+  if (n_st > 1) copy(1, false);
+  copy(0, true);
+  if (n_st > 2) copy(2, false);
+  if (n_st > 1) copy(1, true);
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // (the first stages are waited for whole)
+  barrier();
+  if (n_act > 0) {
+    read_k(0, 0);
+    read_k(0, 2);
+    scores(0);
+    scores(2);
+  }
+  if (gi == 1) barrier();
+  // NOW / NEXT: the wave works on stage n / n + 1 (else it only copies and keeps the barriers)
+  auto stage = [&](int n, auto now_c, auto next_c) __attribute__((always_inline)) {
+    constexpr bool NOW = decltype(now_c)::value, NEXT = decltype(next_c)::value;
+    // ---- vector half
+    if constexpr (NEXT) read_k(n + 1, 0);   // (the other pages' fragments in the matrix half: registers)
+    unsigned ok3 = 0;
+    const bool full = n + 3 < n_st;
+    if (n + 2 < n_st) {
+      if (n + 3 - win0 >= 64 / PF_NP) load_window(n + 2);
+      if (full) {
+        ok3 = stage_ok(n + 3);
+        copy(n + 3, false);
+      }
+      copy(n + 2, true);
+    }
+    const int kb0 = n * PF_KEYS;
+    const bool zero = kb0 + PF_KEYS > kv_total || ok0 != 0xFu;   // the stage holds keys that do not exist
+    if constexpr (NOW) {
+      if (zero || kb0 + PF_KEYS - 1 > ctx + j_first_w) mask(kb0, ok0);
+      softmax();
+    }
+    auto landed = [&]() __attribute__((always_inline)) {   // this wave's copies of K (n + 2) and V (n + 1)
+      if (full)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);
+      else
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+    };
+    if (gi == 1) landed();
+    barrier();
+    // ---- matrix half
+    if constexpr (NOW) {
+      __builtin_amdgcn_s_setprio(1);
+      if constexpr (NEXT) {
+        read_k(n + 1, 2);
+        scores(0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      read_v(n, 0);
+      if constexpr (NEXT) scores(2);
+      __builtin_amdgcn_sched_barrier(0);
+      values(n, 0, ok0, zero);
+      read_v(n, 1);
+      values(n, 1, ok0, zero);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (gi == 0) landed();
+    barrier();
+    ok0 = ok1;
+    ok1 = ok2;
+    ok2 = ok3;
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  int n = 0;
+  for (; n + 1 < n_act; ++n) stage(n, Yes{}, Yes{});
+  if (n < n_act) stage(n++, Yes{}, No{});
+  for (; n < n_st; ++n) stage(n, No{}, No{});
+  if (gi == 0) barrier();
+
+  // ---- the group's tile leaves through LDS as whole rows, 16 bytes per lane
+#pragma unroll
+  for (int rt = 0; rt < PF_R; ++rt) l_run[rt] = pf_sum4(l_run[rt]);
+  constexpr int OPITCH = HD * 2 + 16;
+  static_assert(2 * PF_QT * OPITCH <= 2 * PF_SLOTS_KV * KB, "output staging fits the slots");
+  unsigned char* obuf = lds + gi * (PF_QT * OPITCH);
+#pragma unroll
+  for (int rt = 0; rt < PF_R; ++rt) {
+    const float inv = 1.0f / l_run[rt];
+    unsigned char* orow = obuf + (16 * PF_R * w + 16 * rt + c16) * OPITCH + 8 * r4;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      *reinterpret_cast<uint2*>(orow + 32 * t) = make_uint2(pf_bf16x2(acc[rt][t][0] * inv, acc[rt][t][1] * inv),
+                                                            pf_bf16x2(acc[rt][t][2] * inv, acc[rt][t][3] * inv));
+  }
+  barrier();
+  constexpr int CPR = HD / 8;
+  const int rows = min(PF_QT, T - qbase), tid = tid_wg & (PF_THREADS - 1);
+#pragma unroll
+  for (int i = 0; i < PF_QT * CPR / PF_THREADS; ++i) {
+    const int c = tid + PF_THREADS * i, row = c / CPR, k = c % CPR;
+    const uint4 v = *reinterpret_cast<const uint4*>(obuf + row * OPITCH + 16 * k);
+    if (row < rows)
+      *reinterpret_cast<uint4*>(a.out + int64_t(q_start + qbase + row) * a.o_st + int64_t(h) * a.o_sh + 8 * k) = v;
+  }
+}
+
+// A workgroup of the launch: which body depends on the sequences' own lengths (the caller's max_new and max_kv are upper
+// bounds). Both are modelled as the longer of the longest unit and the CUs' even share, in ns per 64-key stage of a
+// tile -- 2150 / 2 (two key ranges side by side) or 1860 at hd 128, 1500 / 2 or 1450 at hd 64 -- plus 9 or 5 us for each
+// workgroup that a CU runs in turn. Up to a tile per CU the key-range body, which then splits the tiles further, is the faster one.
+// Measured, key ranges / pairs: 3 sequences of 1139 .. 3672 tokens on 627 .. 5751 (16 heads of 128) 368 / 335 us; 8192
+// tokens 298 / 272; 4096 tokens 82 / 125; 5 prompts of 233 .. 876 (14 heads of 64) 29.6 / 24.7; 4096 of them 58 / 101.
+// MANY: the launch may hold that many tiles (prefill_many); without it none of this is in the kernel (0.4 us of a 31 us
+// launch).
+template <int HD, bool MANY>
+__device__ __forceinline__ void prefill_workgroup(const PrefillArgs& a, int bid, unsigned char* lds, unsigned& s_last) {
+  static_assert(2 * PF_SLOTS_KV * PfLds<HD>::K_BYTES <= PF_GROUPS * 2 * PfLds<HD>::STAGE, "the launch's LDS holds the slots");
+  if constexpr (MANY) {   // (at most PF_LANE_SEQS sequences)
+    const int lane = threadIdx.x & 63;
+    PfInfoLanes seqs{0, 0, 0};
+    if (lane < a.n_seqs) seqs = PfInfoLanes{a.info[4 * lane], a.info[4 * lane + 1], a.info[4 * lane + 2]};
+    int tiles = 0, stages = 0, longest = 0;   // over the sequences: tiles, their stages, the most stages of one
+    for (int s = 0; s < a.n_seqs; ++s) {
+      const int T = seqs.n_new(a, s), ctx = seqs.ctx(a, s), nt = (T + PF_QT - 1) / PF_QT;
+      if (T <= 0 || nt > a.tiles_max) continue;
+      tiles += nt;
+      stages += nt * ((ctx + (T + PF_QT) / 2) / PF_KEYS + 1);
+      longest = max(longest, (ctx + T + PF_KEYS - 1) / PF_KEYS);
+    }
+    const int units = tiles * a.n_heads;
+    if (units > PF_CUS) {
+      constexpr int RANGE = HD == 128 ? 2150 : 1500, PAIR = HD == 128 ? 1860 : 1450;
+      const int share = int(int64_t(stages) * a.n_heads / (2 * PF_CUS));   // stages per CU, two at a time
+      const int64_t ranges = int64_t(max(longest / 2, share)) * RANGE + (units + PF_CUS - 1) / PF_CUS * 9000;
+      const int64_t pairs = int64_t(max(longest, share)) * PAIR + (units + 2 * PF_CUS - 1) / (2 * PF_CUS) * 5000;
+      if (pairs < ranges) {
+        prefill_pair_body<HD>(a, seqs, bid, lds);
+        return;
+      }
+    }
+    prefill_body<HD>(a, seqs, bid, lds, s_last);
+  } else {
+    prefill_body<HD>(a, PfInfoMem{}, bid, lds, s_last);
+  }
+}
+
+// Whether a launch's sequences, of at most this many tiles each, may together have more tiles than the GPU has CUs.
+inline bool prefill_many(const PrefillArgs& a) {
+  return a.n_seqs <= PF_LANE_SEQS && int64_t(a.n_seqs) * a.tiles_max * a.n_heads > PF_CUS;
 }
 
 inline size_t pf_align256(size_t x) { return (x + 255) & ~size_t(255); }

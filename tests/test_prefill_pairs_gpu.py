@@ -1,0 +1,113 @@
+"""Chunked-prefill attention in launches of many query tiles, where workgroups take two tiles that share their keys
+(pairs of heads, or of query tiles for an odd number of heads per KV head), against the fp64 product."""
+import pytest
+import torch
+
+from tests.conftest import cpu_gen
+
+pytestmark = pytest.mark.gpu
+
+
+def run_case(n_heads, n_kv, hd, new, ctx, seed, bad_pages=(), poison=True):
+    """Kernel output and reference of sequences with new[i] tokens on ctx[i] cached ones, rows of no sequence between
+    them. bad_pages: (sequence, page) table entries outside the pool, whose tokens are masked. Slots that hold no token
+    are NaN."""
+    from nanoserve_amd.kernels.paged_attention import paged_attention_prefill, prefill_seq_info
+    g = cpu_gen(seed)
+    need = [-(-(a + b) // 16) for a, b in zip(new, ctx)]
+    perm = torch.randperm(sum(need) + 2, generator=g).int()
+    width = max(need)
+    tables = torch.full((len(new), width), int(perm[-1]), dtype=torch.int32)
+    shape = (perm.numel(), 16, n_kv, hd)
+    k, v = (torch.randn(shape, generator=g).bfloat16() for _ in range(2))
+    written = torch.zeros(shape[:2], dtype=torch.bool)
+    at, starts, rows = 0, [], 3
+    for i, n in enumerate(need):
+        tables[i, :n] = perm[at:at + n]
+        at += n
+        total = new[i] + ctx[i]
+        written.view(-1)[(tables[i, :n].long()[:, None] * 16 + torch.arange(16)).view(-1)[:total]] = True
+        starts.append(rows)
+        rows += new[i] + 1
+    q = torch.randn(rows, n_heads, hd, generator=g).bfloat16() * 2
+    if poison:
+        k[~written], v[~written] = float("nan"), float("nan")
+    hidden = {}
+    for i, p in bad_pages:
+        hidden.setdefault(i, []).append(p)
+    dk, dv, dq, dt = k.cuda(), v.cuda(), q.cuda(), tables.clone()
+    for i, p in bad_pages:
+        dt[i, p] = -1 if p % 2 else perm.numel() + 5
+    out = torch.full_like(dq, 7.0)
+    paged_attention_prefill(dq, dk, dv, dt.cuda(), prefill_seq_info(starts, new, ctx, "cuda"), max(new),
+                            max(a + b for a, b in zip(new, ctx)), hd ** -0.5, out=out)
+    ref = torch.full(out.shape, 7.0, dtype=torch.float64, device="cuda")
+    for i, (T, c, r0) in enumerate(zip(new, ctx, starts)):
+        if T == 0:
+            continue
+        pages = tables[i, :need[i]].long().cuda()
+        kk, vv = (t[pages].reshape(-1, n_kv, hd)[:T + c].double() for t in (dk, dv))
+        keys = torch.arange(T + c, device="cuda")
+        see = keys[None] <= c + torch.arange(T, device="cuda")[:, None]
+        for p in hidden.get(i, []):
+            see[:, 16 * p:16 * p + 16] = False
+        for h in range(n_heads):
+            s = (dq[r0:r0 + T, h].double() @ kk[:, h * n_kv // n_heads].t()) * hd ** -0.5
+            w = torch.softmax(s.masked_fill(~see, float("-inf")), -1)
+            ref[r0:r0 + T, h] = w @ vv[:, h * n_kv // n_heads]
+    return out, ref
+
+
+LENS = [500, 1, 129, 640, 255, 128, 700, 384, 257, 0, 512]
+CTXS = [0, 1000, 64, 300, 5, 0, 17, 640, 1, 50, 128]
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(16, 2, 128), (12, 2, 128), (14, 2, 64), (12, 12, 64), (24, 3, 64), (15, 5, 128)])
+def test_ragged_sequences(hiplib, n_heads, n_kv, hd):
+    """P and the output are rounded to bf16 (2^-8 of values of order one, twice); other rows keep what they held."""
+    out, ref = run_case(n_heads, n_kv, hd, LENS, CTXS, seed=n_heads + hd)
+    assert (out.double() - ref).abs().max().item() <= 2e-2
+    assert ((out.double() - ref).norm() / ref.norm()).item() <= 4e-3
+    untouched = (ref == 7.0).all(-1).all(-1)
+    assert untouched.sum() == 3 + len(LENS) and (out[untouched] == 7.0).all()
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(16, 2, 128), (14, 2, 64)])
+def test_long_and_masked_pages(hiplib, n_heads, n_kv, hd):
+    """More than 16 stages (the block-id window moves), pages outside the pool in several places."""
+    bad = [(0, 0), (0, 63), (0, 70), (1, 5), (1, 6), (1, 7), (1, 8), (2, 33)]
+    out, ref = run_case(n_heads, n_kv, hd, [1500, 1311, 900, 1024], [1000, 600, 333, 2100], seed=hd, bad_pages=bad)
+    keep = ~torch.isnan(ref)     # rows whose every key is masked have no value
+    assert torch.equal(torch.isfinite(out)[keep], torch.ones_like(out, dtype=torch.bool)[keep])
+    assert (out.double() - ref)[keep].abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("n_seqs", [40, 64, 65, 90])
+def test_many_sequences(hiplib, n_seqs):
+    """Up to 64 sequences find their tiles over the lanes, more by walking them."""
+    new = [1 + (37 * i) % 400 for i in range(n_seqs)]
+    out, ref = run_case(4, 2, 64, new, [(53 * i) % 200 for i in range(n_seqs)], seed=n_seqs)
+    assert (out.double() - ref).abs().max().item() <= 2e-2
+
+
+def test_same_alone_and_beside_decode_rows(hiplib):
+    """ns_paged_attn_mixed runs the same workgroups: bitwise the prefill rows of the launch without decode rows."""
+    from nanoserve_amd.kernels.paged_attention import paged_attention_mixed, paged_attention_prefill, prefill_seq_info
+    g = cpu_gen(3)
+    new, ctx, nh, nkv, hd = [600, 500, 480], [0, 90, 33], 28, 2, 128
+    nb = sum(-(-(a + b) // 16) for a, b in zip(new, ctx)) + 8
+    perm, width, at = torch.randperm(nb, generator=g).int(), 40, 0
+    tables = torch.zeros(3, width, dtype=torch.int32)
+    for i in range(3):
+        n = -(-(new[i] + ctx[i]) // 16)
+        tables[i, :n] = perm[at:at + n]
+        at += n
+    k, v = (torch.randn(nb, 16, nkv, hd, generator=g).bfloat16().cuda() for _ in range(2))
+    q = torch.randn(4 + sum(new), nh, hd, generator=g).bfloat16().cuda()
+    info = prefill_seq_info([4, 604, 1104], new, ctx, "cuda")
+    dec = perm[at:at + 8].view(4, 2).cuda()
+    lens = torch.tensor([1, 16, 17, 32], dtype=torch.int32).cuda()
+    alone = paged_attention_prefill(q, k, v, tables.cuda(), info, 600, 640, hd ** -0.5, out=torch.zeros_like(q))
+    both = paged_attention_mixed(q, k, v, tables.cuda(), info, 600, 640, dec, lens, torch.arange(4).cuda(), hd ** -0.5,
+                                 out=torch.zeros_like(q))
+    assert torch.equal(alone[4:], both[4:])
