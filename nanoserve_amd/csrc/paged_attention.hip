@@ -925,7 +925,7 @@ __global__ __launch_bounds__(F32_NW * 64) void paged_decode_f32_kernel(
   float m[GC], l[GC], acc[GC][DL];
 #pragma unroll
   for (int h = 0; h < GC; ++h) {
-    m[h] = -INFINITY;
+    m[h] = -3.4028235e38f;   // finite: a wave whose scores are all -inf then weighs 0 beside the others, not NaN
     l[h] = 0.f;
 #pragma unroll
     for (int e = 0; e < DL; ++e) acc[h][e] = 0.f;

@@ -71,6 +71,20 @@ def test_fp32_rows_ignore_what_lies_past_the_context(hiplib):
     assert (out.double() - clean).abs().max().item() <= 1e-5
 
 
+def test_fp32_rows_with_scores_of_minus_infinity(hiplib):
+    """Keys that a query can't see at all (a score of -inf), for a whole 64-token chunk of one wave and of a row's later
+    half: they weigh nothing."""
+    from nanoserve_amd.kernels.paged_attention import paged_attention_decode
+    lens = [128, 300, 700]
+    q, k, v, tables, cl = case(14, 2, 64, lens, torch.float32, 6)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    for b, lo, hi in ((0, 64, 128), (1, 192, 300), (2, 320, 640)):
+        for t in range(lo, hi):
+            k[tables[b, t // 16].long(), t % 16, :, 0] = -float("inf")
+    out = paged_attention_decode(q.cuda(), k.cuda(), v.cuda(), tables.cuda(), cl.cuda(), 0.125).cpu()
+    assert (out.double() - reference(q, k, v, tables, cl, 0.125)).abs().max().item() <= 1e-5
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,width", [(16, 2, 128, 1024), (16, 2, 128, 1025), (12, 2, 128, 2048), (14, 2, 64, 1025),
                                                    (14, 2, 64, 2049), (16, 1, 128, 2048)])
 def test_wide_tables(hiplib, n_heads, n_kv, hd, width):
