@@ -1841,7 +1841,6 @@ struct TgPlan {
 // 96 60; 512 rows of it: 128 x 96 tiles 57, 34, 28, 26 us in 1 .. 4 slices, 128 x 128 in 5 27). Plain,
 // residual and RoPE products of one shape take the same slices, so their sums agree bit for bit; SiLU products are not
 // sliced. A function of the shape alone, so a given call always sums in the same order.
-static inline void tg_plan_override(TgPlan&, int, int, int) {}
 static TgPlan tg_plan_of(int M, int N, int K, int epi, int sp_min, int sp_max) {
   const bool silu = epi == EPI_SILU;
   const int T = target_workgroups(), slabs = (K + TG_BK - 1) / TG_BK;
@@ -1871,7 +1870,6 @@ static TgPlan tg_plan(int M, int N, int K, int epi) {
   // (128 x 96 tiles, the only ones that RoPE's heads do not fit, are the smallest: any other tile keeps within the round)
   if (epi == EPI_ROPE) p = tg_plan_of(M, N, K, epi, p.splits, p.splits);
   const int slabs = (K + TG_BK - 1) / TG_BK;
-  tg_plan_override(p, M, N, epi);
   p.splits = (slabs + p.kps - 1) / p.kps;   // every slice non-empty
   if (p.splits > 1)
     p.bytes = G_CNT_BYTES + align256(sizeof(float) * size_t(p.tiles_m) * p.tiles_n * p.splits * TG_TILE[p.shape].bm * TG_TILE[p.shape].bn);
@@ -1888,6 +1886,7 @@ static TgArgs tg_args(const void* x, const void* w, const void* bias, void* y, i
   a.K = K;
   return a;
 }
+constexpr int TG_WS_K = 4096;
 // a: operands, shape and (ROPE) the epilogue's fields; the plan fills the rest
 template <int EPI>
 static int launch_tiled(TgArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
@@ -1895,7 +1894,10 @@ static int launch_tiled(TgArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
   // 32-bit buffer offsets: every row offset of X and W (plus a tile's overhang) must fit
   NS_REQUIRE((int64_t(M) + 256) * K * 2 < (int64_t(1) << 31) && (int64_t(N) + 256) * K * 2 < (int64_t(1) << 31),
              "gemm: X [%d, %d] or W [%d, %d] too large for 32-bit buffer offsets", M, K, N, K);
-  const TgPlan p = tg_plan(M, N, K, EPI);
+  TgPlan p = tg_plan(M, N, K, EPI);
+  // Without a workspace: unsliced, below the K from which a workspace has always been asked for. (A caller that records
+  // such a product as its first call on the device can't allocate one.)
+  if (ws == nullptr && p.splits > 1 && K < TG_WS_K) p = tg_plan_of(M, N, K, EPI, 1, 1);
   a.tiles_m = p.tiles_m;
   a.tiles_n = p.tiles_n;
   a.splits = p.splits;
@@ -1954,7 +1956,11 @@ static size_t skinny_large_m_bytes(const Plan& p, int mblocks) {
 extern "C" size_t ns_gemm_workspace_bytes(int M, int N, int K) {
   if (M < 1 || N < 1 || K < 32) return 0;
   if (M > G_MAX_M) {
-    size_t a = tg_plan(M, N, K, EPI_STORE).bytes;   // only plain and residual products are sliced, and alike
+    // plain and residual products are sliced alike; RoPE's (whole heads: N a multiple of 64) in as many slices, but of
+    // 128-wide tiles where those take 128 x 96, so its padded partials can be larger
+    size_t a = tg_plan(M, N, K, EPI_STORE).bytes;
+    const size_t r = N % 64 == 0 ? tg_plan(M, N, K, EPI_ROPE).bytes : 0;
+    a = a > r ? a : r;
     // the 64-row token blocks of the skinny kernel (STORE with long K; residual + statistics at any K)
     if (M <= t16_max_m() && (M + G_MAX_M - 1) / G_MAX_M * ((N + 63) / 64) <= G_MAX_TILES) {
       const size_t c = skinny_large_m_bytes(make_plan((N + 63) / 64, K), (M + G_MAX_M - 1) / G_MAX_M);

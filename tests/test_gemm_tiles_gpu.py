@@ -73,3 +73,39 @@ def test_rope(hiplib, M, nh, nkv, hd, K):
             assert torch.equal(a, r)
         if cached:
             assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
+
+
+def test_rope_slices_of_wider_tiles_than_the_plain_product(hiplib):
+    """A merged QKV of 192 columns runs 128-wide RoPE tiles (two, the second half empty) where the plain product takes
+    two of 96: its K slices' partials need the larger workspace that ns_gemm_workspace_bytes now names."""
+    from nanoserve_amd import _lib
+    from nanoserve_amd.kernels.fused import rope_qkv
+    from nanoserve_amd.kernels.linear import linear
+    L = _lib.lib()
+    M, hd, K, N = 564, 64, 4096, 192
+    x, w = (t.cuda() for t in operands(M, N, K, seed=31))
+    cos, sin = (t.cuda() for t in ops.rope_tables(torch.arange(M), hd, 1e6, BF))
+    ws = torch.zeros(L.ns_gemm_workspace_bytes(M, N, K), dtype=torch.uint8, device="cuda")
+    out = [torch.empty(M, 1, hd, dtype=BF, device="cuda") for _ in range(3)]
+    rc = L.ns_gemm_rope_qkv(x.data_ptr(), w.data_ptr(), None, cos.data_ptr(), sin.data_ptr(), *(t.data_ptr() for t in out),
+                            None, None, None, M, K, 1, 1, hd, 1, None, None, 0.0, ws.data_ptr(), ws.numel(), _lib.stream_of(x))
+    assert rc == 0, L.ns_last_error()
+    for a, r in zip(out, rope_qkv(linear(x, w), cos, sin, 1, 1, hd)):
+        assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 1032, 2080), (512, 1536, 1536), (1003, 896, 4064)])
+def test_short_k_without_a_workspace(hiplib, M, N, K):
+    """Products of K < 4096 run unsliced where the caller has no workspace; longer ones are refused."""
+    from nanoserve_amd import _lib
+    L = _lib.lib()
+    x, w = operands(M, N, K, seed=32)
+    dx, dw = x.cuda(), w.cuda()
+    y = torch.empty(M, N, dtype=BF, device="cuda")
+    assert L.ns_gemm_workspace_bytes(M, N, K) > 0
+    rc = L.ns_gemm(dx.data_ptr(), dw.data_ptr(), None, y.data_ptr(), M, N, K, 1, None, None, 0.0, None, 0, _lib.stream_of(dx))
+    assert rc == 0, L.ns_last_error()
+    rows = edge_rows(M)
+    bf16_check(y.cpu()[rows], ref_linear(x[rows], w), f"unsliced {M} x {N} x {K}", dot_bound(x[rows], w))
+    rc = L.ns_gemm(dx.data_ptr(), dw.data_ptr(), None, y.data_ptr(), 256, 512, 8960, 1, None, None, 0.0, None, 0, _lib.stream_of(dx))
+    assert rc != 0
