@@ -296,9 +296,11 @@ size_t ns_gemm_workspace_bytes(int M, int N, int K);
  * Any M >= 1: above 64 rows (prefill chunks, mixed steps, speculative verify batches; nanoserve/model.py:231,
  * 256-257 on the large-token path) x_sumsq must be NULL (materialise a normalised input with
  * ns_rms_norm_apply first). Up to 192 rows a projection with K <= 2048 and at most 8,192 rows of W runs on the
- * tile-16 kernel in 16-token blocks; otherwise a tiled MFMA kernel computes the product (tiles of 128 x 96 to
+ * tile-16 kernel in 16-token blocks (at most 1,024 of them), one with longer K on the skinny kernel in 64-row blocks
+ * while these read at most 2^25 weights in all; otherwise a tiled MFMA kernel computes the product (tiles of 128 x 96 to
  * 256 x 256 outputs, K sliced and the slices summed in a fixed order for long K and few tiles), its
- * workspace sized by ns_gemm_workspace_bytes(M, N, K) as for the skinny kernels.
+ * workspace sized by ns_gemm_workspace_bytes(M, N, K) as for the skinny kernels (where the tiled kernel runs and
+ * K < 4096, workspace may be NULL: the product then runs unsliced).
  */
 int ns_gemm(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int dtype,
             const float* x_sumsq, const void* x_norm_w, float x_eps,

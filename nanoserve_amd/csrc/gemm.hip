@@ -1713,12 +1713,29 @@ static bool t16_token_split(int M, int tiles) {
 }
 // Above 64 rows a plain input on a projection the tile-16 kernel takes (K <= 2048, at most T16_MAX_TILES
 // tiles) runs it token-split (16-token blocks, the blocks of a tile re-reading its weights from L2), in as
-// many rounds as it needs, up to T16_LARGE_M rows (speculative verify batches); larger chunks go to the
-// tiled kernel.
+// many rounds as it needs, up to T16_LARGE_M rows (speculative verify batches); larger chunks, and those that
+// tg_large_m names, go to the tiled kernel.
 constexpr int T16_LARGE_M = 192;
 constexpr int t16_max_m() { return T16_LARGE_M; }
 static bool t16_large_m(int M, int K, int tiles, bool normed) {
   return M > G_MAX_M && M <= (normed ? G_NORM_ROWS : t16_max_m()) && tile16_fits(K, tiles);
+}
+// Plain products of 65 .. T16_LARGE_M rows that the tiled kernel takes. The tile-16 kernel's time grows with its
+// workgroups (about 8.5 ns each over 3.5 us), the skinny kernel's with the weights that its 64-row blocks read in all; the
+// tiled kernel's hardly grows with the rows (one or two row tiles). Tile-16 / tiled, graph replays over cold weights, us:
+// 2048 x 1536 at 128 rows (1024 workgroups) 11.7 / 12.8, at 144 (1152) 13.6 / 12.9, at 192 16.0 / 13.0; 2560 x 2048 at 96
+// (960) 12.5 / 13.0, at 120 (1280) 14.8 / 13.1, at 192 21.3 / 14.7; 1536 x 1536 at 160 (960) 11.4 / 12.3, at 192 (1152) 13.5 /
+// 12.4. Skinny / tiled: 1536 x 8960 at 120 rows (28 M elements read) 23.0 / 22.9, at 144 (41 M) 25.0 / 21.7, at 192 30.3 /
+// 21.8; 2048 x 11008 at 96 (45 M) 28.3 / 24.7, at 192 44.8 / 27.2; 896 x 4864 at 160 (13 M) 14.4 / 16.9.
+constexpr int T16_LARGE_WG = 1024;
+constexpr int64_t SKINNY_LARGE_ELEMS = int64_t(1) << 25;
+static bool tg_fits(int M, int N, int K) {   // 32-bit buffer offsets: every row offset of X and W (plus a tile's overhang)
+  return (int64_t(M) + 256) * K * 2 < (int64_t(1) << 31) && (int64_t(N) + 256) * K * 2 < (int64_t(1) << 31);
+}
+static bool tg_large_m(int M, int N, int K) {
+  if (M <= G_MAX_M || M > t16_max_m() || !tg_fits(M, N, K)) return false;
+  if (tile16_fits(K, (N + 15) / 16)) return (M + 15) / 16 * ((N + 15) / 16) > T16_LARGE_WG;
+  return int64_t(N) * K * ((M + G_MAX_M - 1) / G_MAX_M) > SKINNY_LARGE_ELEMS;
 }
 template <int EPI, bool NX>
 static void launch_t16_nx(const GemmArgs& a, int tiles, hipStream_t st) {
@@ -1891,20 +1908,20 @@ constexpr int TG_WS_K = 4096;
 template <int EPI>
 static int launch_tiled(TgArgs a, void* ws, size_t ws_bytes, hipStream_t st) {
   const int M = a.M, N = a.N, K = a.K;
-  // 32-bit buffer offsets: every row offset of X and W (plus a tile's overhang) must fit
-  NS_REQUIRE((int64_t(M) + 256) * K * 2 < (int64_t(1) << 31) && (int64_t(N) + 256) * K * 2 < (int64_t(1) << 31),
+  NS_REQUIRE(tg_fits(M, N, K),
              "gemm: X [%d, %d] or W [%d, %d] too large for 32-bit buffer offsets", M, K, N, K);
   TgPlan p = tg_plan(M, N, K, EPI);
-  // Without a workspace: unsliced, below the K from which a workspace has always been asked for. (A caller that records
+  // Without a workspace (or with one too small): unsliced, below the K from which a workspace has always been asked for. (A caller that records
   // such a product as its first call on the device can't allocate one.)
-  if (ws == nullptr && p.splits > 1 && K < TG_WS_K) p = tg_plan_of(M, N, K, EPI, 1, 1);
+  const bool ws_ok = ws != nullptr && ws_bytes >= p.bytes && reinterpret_cast<uintptr_t>(ws) % 256 == 0;
+  if (p.splits > 1 && K < TG_WS_K && !ws_ok) p = tg_plan_of(M, N, K, EPI, 1, 1);
   a.tiles_m = p.tiles_m;
   a.tiles_n = p.tiles_n;
   a.splits = p.splits;
   a.kps = p.kps;
   if (p.splits > 1) {
     NS_REQUIRE(p.tiles_m * p.tiles_n <= G_MAX_TILES, "gemm: %d tiles exceed the counter region", p.tiles_m * p.tiles_n);
-    if (ws == nullptr || ws_bytes < p.bytes || reinterpret_cast<uintptr_t>(ws) % 256 != 0) {
+    if (!ws_ok) {
       set_error("gemm: a zero-initialised, 256-byte aligned workspace of %zu bytes is needed, got %zu", p.bytes,
                 ws == nullptr ? size_t(0) : ws_bytes);
       return NS_E_WORKSPACE;
@@ -1978,7 +1995,8 @@ extern "C" int ns_gemm(const void* x, const void* w, const void* bias, void* y, 
   if (st != NS_OK) return st;
   NS_REQUIRE(y != nullptr && aligned16(y), "gemm: output must be 16-byte aligned");
   if (M > G_MAX_M) {
-    if (t16_large_m(M, K, (N + 15) / 16, x_sumsq != nullptr)) {
+    const bool tiled = x_sumsq == nullptr && tg_large_m(M, N, K);
+    if (!tiled && t16_large_m(M, K, (N + 15) / 16, x_sumsq != nullptr)) {
       GemmArgs a = base_args(x, w, M, N, K);
       a.bias = static_cast<const bf16_t*>(bias);
       a.y = static_cast<bf16_t*>(y);
@@ -1987,7 +2005,7 @@ extern "C" int ns_gemm(const void* x, const void* w, const void* bias, void* y, 
     }
     NS_REQUIRE(x_sumsq == nullptr, "gemm: a normalised input (x_sumsq) above %d rows needs K <= %d and at most %d "
                                    "rows", G_MAX_M, T16_MAX_K, G_NORM_ROWS);
-    if (skinny_large_m(M, K, N)) {
+    if (!tiled && skinny_large_m(M, K, N)) {
       GemmArgs a = base_args(x, w, M, N, K);
       a.bias = static_cast<const bf16_t*>(bias);
       a.y = static_cast<bf16_t*>(y);
@@ -2134,7 +2152,8 @@ extern "C" int ns_gemm_rope_qkv(const void* x, const void* w, const void* bias, 
   NS_REQUIRE(aligned16(cos) && aligned16(sin) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(k_cache) &&
                  aligned16(v_cache),
              "gemm_rope_qkv: operands must be 16-byte aligned");
-  if (M > G_MAX_M && !t16_large_m(M, K, N / 16, x_sumsq != nullptr)) {
+  const bool tiled = x_sumsq == nullptr && (bias == nullptr || aligned16(bias)) && tg_large_m(M, N, K);
+  if (M > G_MAX_M && (tiled || !t16_large_m(M, K, N / 16, x_sumsq != nullptr))) {
     TgArgs t = tg_args(x, w, bias, nullptr, M, N, K);
     t.cosb = static_cast<const bf16_t*>(cos);
     t.sinb = static_cast<const bf16_t*>(sin);

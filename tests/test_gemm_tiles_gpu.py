@@ -109,3 +109,33 @@ def test_short_k_without_a_workspace(hiplib, M, N, K):
     bf16_check(y.cpu()[rows], ref_linear(x[rows], w), f"unsliced {M} x {N} x {K}", dot_bound(x[rows], w))
     rc = L.ns_gemm(dx.data_ptr(), dw.data_ptr(), None, y.data_ptr(), 256, 512, 8960, 1, None, None, 0.0, None, 0, _lib.stream_of(dx))
     assert rc != 0
+
+
+# both sides of the rows at which the tile-16 kernel's 16-token blocks (1,024 in all) and the skinny kernel's 64-row blocks
+# (2^25 weights read in all) give way to the tiled kernel
+@pytest.mark.parametrize("M,N,K", [(128, 2048, 1536), (129, 2048, 1536), (192, 1536, 1536), (97, 2560, 2048), (65, 8185, 96),
+                                   (128, 1536, 8960), (129, 1536, 8960), (65, 2048, 11008), (192, 1003, 8992)])
+def test_verify_rows_at_the_kernels_crossover(hiplib, M, N, K):
+    from nanoserve_amd.kernels.linear import linear
+    x, w = operands(M, N, K, seed=M + N + 1)
+    b = (torch.randn(N, generator=cpu_gen(5)) * 0.1).to(BF)
+    dx, dw = x.cuda(), w.cuda()
+    for bias in (None, b):
+        y = linear(dx, dw, None if bias is None else bias.cuda())
+        bf16_check(y.cpu(), ref_linear(x, w, bias), f"{M} x {N} x {K}", dot_bound(x, w))
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K", [(128, 12, 2, 128, 1536), (129, 12, 2, 128, 1536), (120, 16, 2, 128, 2048),
+                                           (192, 14, 2, 64, 896), (65, 120, 4, 64, 96)])
+def test_verify_rope_at_the_kernels_crossover(hiplib, M, nh, nkv, hd, K):
+    """The merged projection takes the plain one's kernel: the same bits."""
+    from nanoserve_amd.kernels.fused import rope_qkv
+    from nanoserve_amd.kernels.linear import linear, linear_rope_qkv
+    N = (nh + 2 * nkv) * hd
+    x, w = (t.cuda() for t in operands(M, N, K, seed=M + hd))
+    g = cpu_gen(M)
+    b = (torch.randn(N, generator=g) * 0.1).to(BF).cuda()
+    cos, sin = (t.cuda() for t in ops.rope_tables(torch.randint(0, 32768, (M,), generator=g), hd, 1e6, BF))
+    fused = linear_rope_qkv(x, w, b, cos, sin, nh, nkv, hd, None, None, None)
+    for a, r in zip(fused, rope_qkv(linear(x, w, b), cos, sin, nh, nkv, hd, None, None, None)):
+        assert torch.equal(a, r)
